@@ -144,6 +144,15 @@ TCFP_DEV void dma16_nt(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
                : "memory");
 }
 
+// One byte per lane from rsrc + voff + soff, zero-extended, into the 32-bit
+// LDS word lds + 4 * lane.
+TCFP_DEV void dma1(v4i rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("buffer_load_ubyte %0, %1, %2 offen lds"
+               :
+               : "v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds)
+               : "memory");
+}
+
 // 16 bytes from a per-lane global address into LDS at lds + 16 * lane
 // (lds wave-uniform); counted by vmcnt like dma16.
 TCFP_DEV void gdma16(const void* src, uint32_t lds) {
@@ -292,7 +301,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   constexpr int DI = RPW / 8;       // 1 KiB DMA instructions per wave and stage
   static_assert(RPW % 16 == 0 && BM % RPW == 0 && BN % RPW == 0, "DMA rows must tile regions");
   static_assert(MB >= 1 && NB >= 1, "tile too small for the wave grid");
-  static_assert(NS == 2 || (NS == 4 && SCALE == 0), "deep pipelines carry no exponent loads");
+  static_assert(NS == 2 || (NS == 4 && (SCALE == 0 || (SCALE == 1 && AQ == 0 && NW == 4))),
+                "deep pipelines: per-tensor scales, or block exponents on four waves");
   static_assert(SCALE != 2 || (NW == 4 && BM == 128 && BN == 64 && NS == 2),
                 "fp32 block scales use the 128 x 64 tile");
   // SCALE 2: a three-slot ring of per-stage fp32 scale areas (up to four
@@ -302,9 +312,18 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // block of the stage][row] (a block of bs >= 32 columns fills
   // kSK / bs of the four slots)
   constexpr int kExB = AQ ? 2 * (kSK / 32) * BM : 0;
+  // block exponents of the deep pipeline: one byte per (32-column K block,
+  // stage row) of each buffered stage, brought in with the stage's operands.
+  // The byte loads below write one 32-bit LDS word per lane.
+  constexpr bool kExLds = SCALE == 1 && NS == 4;
+  constexpr int kExRows = BM + 2 * BN;               // 64 rows per wave
+  constexpr int kExStage = kExLds ? (kSK / 32) * kExRows * 4 : 0;
+  constexpr int EI = kExLds ? kSK / 32 : 0;          // byte loads per wave and stage
+  static_assert(!kExLds || (kExRows == NW * 64 && BM % 64 == 0 && BN == 64),
+                "each wave brings in 64 rows' exponents");
   // AQ: per-wave scratch of one float per (row, block) segment of a stage
   constexpr int kAqS = AQ ? NW * (BM / NW) * (kSK >> F32BS) * 4 : 0;
-  __shared__ __align__(16) uint8_t lds[NS * STAGE + 3 * kScB + kExB + kAqS];
+  __shared__ __align__(16) uint8_t lds[NS * STAGE + 3 * kScB + kExB + kAqS + NS * kExStage];
 
   const int M = g.M, N = g.N;
   int K = g.K;
@@ -401,6 +420,43 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
       uint32_t(reinterpret_cast<uintptr_t>((TCFP_LDS uint8_t*)lds)) + uint32_t(NS * STAGE);
   const int nkb = SCALE == 2 ? (K >> f32_bsh) : 0;
 
+  // ---- block exponents of the deep pipeline.  Loaded into registers ahead
+  // of use (load_raw), their waits would drain the operand DMAs issued
+  // behind them, stage by stage; in LDS they are one more DMA.  Wave w brings in those of
+  // stage rows 64 w .. + 63 (one array, one row per lane; rows past the
+  // matrix read 0), K block by K block.  Byte loads: an exponent array's
+  // rows start at any alignment (M, N are any numbers).
+  v4i exrsrc = {};
+  uint32_t exvoff = kOob, exlds = 0;
+  int exld = 0;
+  if constexpr (kExLds) {
+    const int er = wave * 64;
+    const int8_t* eb;
+    int base, rows;
+    if (er < BM) {
+      eb = g.e_a; base = m0 + er; rows = M;
+    } else if (er < BM + BN) {
+      eb = g.e_0; base = n0; rows = N;
+    } else {
+      eb = SPLIT ? g.e_0 : g.e_1; base = n1; rows = N;
+    }
+    exld = rows;
+    exrsrc = make_rsrc(eb, uint32_t(int64_t(K >> g.bs_shift) * rows));
+    exvoff = base + lane < rows ? uint32_t(base + lane) : kOob;
+    exlds = uint32_t(reinterpret_cast<uintptr_t>((TCFP_LDS uint8_t*)lds)) +
+            uint32_t(NS * STAGE) + uint32_t(er) * 4;
+  }
+  // K block b (32 columns) of stage t -> the stage's exponent slots
+  auto issue_ex = [&](int t, int b) {
+    if constexpr (kExLds) {
+      const int k = t * kSK + b * 32;
+      const bool in = k < K;
+      const uint32_t soff = uint32_t(in ? k >> g.bs_shift : 0) * uint32_t(exld);
+      dma1(exrsrc, in ? exvoff : kOob, soff,
+           exlds + uint32_t(t & (NS - 1)) * kExStage + uint32_t(b * kExRows * 4));
+    }
+  };
+
   // DMA of stage t (K columns t*128 ..) into buffer t & 1.  Stages past the
   // end are issued as all-out-of-range loads (zeros into a buffer nobody
   // reads again), so the issue stays branch-free.
@@ -418,6 +474,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
       const int c = (i & 1) ? chunk1 : chunk0;
       dma16(rsrc, (!live || (last && c * 16 >= krem)) ? kOob : voff[i], soff, dst + i * 1024);
     }
+#pragma unroll
+    for (int b = 0; b < EI; ++b) issue_ex(t, b);
     if constexpr (SCALE == 2) {
       if (live && wave < (kSK >> f32_bsh)) {
         const int kb = min(((t * kSK) >> f32_bsh) + wave, nkb - 1);
@@ -627,7 +685,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // Raw exponents of stage t, one register per (fragment, sub-step); rows
   // or K past the matrix read as 0 (2^0, multiplying zero operands).
   auto load_raw = [&](int* raw, int t) {
-    if constexpr (SCALE == 1) {
+    if constexpr (SCALE == 1 && !kExLds) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const int k = t * kSK + h * 64 + lg * 32;
@@ -652,10 +710,22 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // byte 0 of the VGPR (the MFMA's opsel does not select other bytes), so
   // each sub-step gets its own register.
   auto pack = [&](uint32_t* sc, const int* raw) {
-    if constexpr (SCALE == 1) {
+    if constexpr (SCALE == 1 && !kExLds) {
 #pragma unroll
       for (int f = 0; f < 2 * (NF + MB); ++f) sc[f] = e8m0_of(raw[f]);
     }
+  };
+
+  // The deep pipeline's codes of fragment x (weights, then activations) for
+  // sub-step h of stage t, from the stage's exponent slots: of the raw byte
+  // u, u ^ 128 = e + 128, so the E8M0 code is that minus 1, at least 0.
+  auto ex_code = [&](int t, int h, int x) -> uint32_t {
+    const int row = x < NF ? BM + (x / NB) * BN + wn * TNW + (x % NB) * 32 + lr
+                           : wm * TMW + (x - NF) * 32 + lr;
+    const uint32_t u = *reinterpret_cast<const uint32_t*>(
+        lds + NS * STAGE + (t & (NS - 1)) * kExStage + ((2 * h + lg) * kExRows + row) * 4);
+    const uint32_t v = u ^ 128u;
+    return (v > 1u ? v : 1u) - 1u;
   };
 
   // [slot][n-block][m-block].  Block-scaled dual GEMMs keep one set: with
@@ -757,9 +827,9 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // touch no memory, so without it they drift past the barrier and the LDS
   // reads before it are left with nothing to hide behind.
   // With NS stages, the DMAs of stages t+2 .. t+NS-1 may stay in flight.
-  constexpr int kInflight = (NS - 2) * DI;
+  constexpr int kInflight = (NS - 2) * (DI + EI);
   // four stages in flight on one four-wave workgroup per CU
-  constexpr bool kDeep = NW == 4 && NS == 4 && SCALE == 0 && AQ == 0;
+  constexpr bool kDeep = NW == 4 && NS == 4 && SCALE != 2 && AQ == 0;
   auto sync_all = [&]() {
     __builtin_amdgcn_sched_barrier(0);
     // vmcnt(kInflight) lgkmcnt(0), expcnt untouched
@@ -789,7 +859,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
       // (the exponent loads were issued before all of them and are complete;
       // a wave that also loads fp32 scales issues one more per stage, which
       // only makes this wait longer)
-      constexpr int kPro = (NS - 1) * DI;
+      constexpr int kPro = (NS - 1) * (DI + EI);
       __builtin_amdgcn_s_waitcnt((kPro & 15) | (7 << 4) | ((kPro >> 4) << 14));
     }
     __builtin_amdgcn_s_barrier();
@@ -798,6 +868,12 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
     pack(sc, raw);
     read_frags(f0, 0, 0);
     if constexpr (kDeep) read_frags(f1, 0, 1);
+    if constexpr (kExLds) {
+#pragma unroll
+      for (int x = 0; x < NF + MB; ++x)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) sc[2 * x + h] = ex_code(0, h, x);
+    }
   }
   if constexpr (SCALE == 2) {
     // Per K-block partial products p (fresh accumulators), folded into acc
@@ -929,13 +1005,14 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
     constexpr int RSL = 5;        // slots after the barrier that carry the reads
     static_assert(1 + DSL <= SL && 1 + RSL < SL, "deep schedule slots");
     v8i g0[NFR], g1[NFR];
+    uint32_t sg[2 * NFR];  // the other stage's E8M0 codes (block exponents)
     // chunks past K in the last stage (per lane, even / odd DMA instruction)
     const bool tail0 = chunk0 * 16 >= krem, tail1 = chunk1 * 16 >= krem;
     // stage t on fragments c (sub-steps 0 / 1); stage t + 1's read into x
-    auto stage = [&](v8i* c0, v8i* c1, v8i* x0, v8i* x1, int t) {
+    auto stage = [&](v8i* c0, v8i* c1, v8i* x0, v8i* x1, const uint32_t* cs, uint32_t* xs, int t) {
       auto mf = [&](int s) {
         const int h = s / NP, idx = s % NP;
-        mfma1(h ? c1 : c0, sc, h, idx % NF, idx / NF);
+        mfma1(h ? c1 : c0, cs, h, idx % NF, idx / NF);
       };
       // fragment r of stage t + 1 (sub-step r / NFR)
       auto rd = [&](int r) {
@@ -944,6 +1021,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
         const int rb = x < NF ? (BM + (x / NB) * BN + wn * TNW + (x % NB) * 32) * kRowB
                               : (wm * TMW + (x - NF) * 32) * kRowB;
         (h ? x1 : x0)[x] = make_frag(lds_read16(st, rb + ro[h][0]), lds_read16(st, rb + ro[h][1]));
+        if constexpr (kExLds) xs[2 * x + h] = ex_code(t + 1, h, x);
       };
       mf(0);
       __builtin_amdgcn_sched_barrier(0);
@@ -974,6 +1052,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
 #pragma unroll
           for (int i = j * DI / DSL; i < (j + 1) * DI / DSL; ++i)
             dma16(rsrc, vo[i], soff, dst + i * 1024);
+#pragma unroll
+          for (int b = j * EI / DSL; b < (j + 1) * EI / DSL; ++b) issue_ex(tr, b);
         }
         if (j < RSL) {
 #pragma unroll
@@ -984,8 +1064,8 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
     };
     // two stages per trip: the fragment sets swap roles
     for (int t = 0; t < nt; t += 2) {
-      stage(f0, f1, g0, g1, t);
-      if (t + 1 < nt) stage(g0, g1, f0, f1, t + 1);
+      stage(f0, f1, g0, g1, sc, sg, t);
+      if (t + 1 < nt) stage(g0, g1, f0, f1, sg, sc, t + 1);
     }
   } else {
   for (int t = 0; t < nt; ++t) {
@@ -2014,6 +2094,15 @@ int num_cus() {
   return n;
 }
 
+// Block exponents on the small tile: whether a one-round grid takes the
+// four-stage pipeline, whose longer prologue needs some stages to pay
+// (two-stage -> four-stage, block 64: 128 x 2048 x 128 5.2 -> 5.7 us, 256 x
+// 1024 x 256 5.8 -> 6.1, 512 x 512 x 384 6.7 -> 6.4, 1000 x 1024 x 512 8.7 ->
+// 7.7, 1000 x 1024 x 1024 13.1 -> 9.6, 333 x 2048 x 2048 21.6 -> 13.2, 64 x
+// 4096 x 4096 37.4 -> 18.9, 16 x 16384 x 4096 48.5 -> 24.1).  With few tiles
+// the gain starts later.
+bool deep_exps(int64_t tiles, int64_t k) { return k >= 640 || (k >= 384 && tiles >= 32); }
+
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // The persistent large-tile launch: full 256 x 128 tiles, two K stages at
@@ -2089,13 +2178,17 @@ int launch_gemm(GemmArgs ga, hipStream_t st) {
     const dim3 grid(unsigned(ga.tiles_m) * unsigned(ga.tiles_n), splits);
     // a small-tile launch that fits in one round gets the 4-stage pipeline
     // (one workgroup per CU, 128 KiB of LDS)
-    const bool deep = SCALE == 0 && small && int64_t(grid.x) * splits <= num_cus();
+    // (block exponents: 32-bit offsets into the exponent arrays)
+    bool deep = SCALE != 2 && small && int64_t(grid.x) * splits <= num_cus();
+    if (SCALE == 1 &&
+        (!deep_exps(grid.x, k) || int64_t(k >> ga.bs_shift) * std::max(m, n) >= kMaxSpan))
+      deep = false;
     if (small && deep) {
-      if constexpr (SCALE == 0) {
-        // (the eight-wave tuning policy serves FP8 operands; bf16 takes the
-        // four-wave tile under every policy)
-        if (AF != kBF16 && g_tile_policy == 3) {
-          if constexpr (AF != kBF16)
+      if constexpr (SCALE != 2) {
+        // (the eight-wave tuning policy serves FP8 operands with per-tensor
+        // scales; the others take the four-wave tile under every policy)
+        if (SCALE == 0 && AF != kBF16 && g_tile_policy == 3) {
+          if constexpr (SCALE == 0 && AF != kBF16)
             gemm_nt_dma_kernel<AF, BF, SPLIT, OutT, 8, 128, 64, SCALE, 4><<<grid, 512, 0, st>>>(ga);
         } else
           gemm_nt_dma_kernel<AF, BF, SPLIT, OutT, 4, 128, 64, SCALE, 4><<<grid, 256, 0, st>>>(ga);
