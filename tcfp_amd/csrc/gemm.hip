@@ -2068,6 +2068,161 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
   }
 }
 
+// ---------------------------------------------------------------------------
+// Few activation rows (M <= 64): the weight stream
+// ---------------------------------------------------------------------------
+//
+// With few rows the product is bound by reading the weight codes once; the
+// tiles above put them on ceil(N / 64) workgroups that each walk K in series
+// behind a barrier per 128 columns.  Here a workgroup owns 16 output columns
+// and its eight waves split K between them: a wave reads its weight rows
+// straight into MFMA fragments (16x16x128: 16 rows x 128 bytes per step, no
+// LDS, no barrier), kSkU steps of both slots in flight at a time, so a CU
+// with two workgroups keeps 256 KiB of loads outstanding.  The waves' partial
+// sums meet in LDS and are added in wave order (deterministic).
+// MT activation tiles of 16 rows (rows past M read as zero).
+// Measured against the tiles (graph replays over operand sets beyond L2;
+// M x N x K, bf16 out, before -> after): per tensor 1 x 1024 x 1024 6.3 ->
+// 4.0 us, 16 x 4096 x 4096 15.8 -> 9.0 us (3.7 TB/s of weight codes), 32 x
+// 4096 x 4096 16.7 -> 11.7 us, 64 x 1024 x 1024 7.1 -> 6.1 us; block 64 16 x
+// 4096 x 4096 44.3 -> 11.9 us (18.6 on the four-stage tile).  Bound: the
+// stream's latency at these sizes (a launch, ~1 us to the first bytes, the
+// LDS sum).  Wider column tiles (32 or 64 per workgroup) lost at N <= 8192;
+// non-temporal weight loads and loads pinned ahead of the products measured
+// level or slower.
+constexpr int kSkWaves = 8;
+constexpr int kSkN = 16;   // output columns per workgroup
+
+// Fragment layout: lane l holds row l % 16 and, of the step's eight 16-byte
+// chunks, chunks l / 16 and 4 + l / 16 (in both operands); the E8M0 scale of
+// lane l covers the 32-column K block l / 16 of its row.
+template <int AF, int BF, bool SPLIT, typename OutT, int SCALE, int MT>
+__global__ __launch_bounds__(kSkWaves * 64, MT == 4 ? 2 : 4) void gemm_skinny_kernel(GemmArgs g) {
+  constexpr int NSL = SPLIT ? 1 : 2;                     // weight slots
+  constexpr int U = MT == 1 ? 4 : 2;                     // steps in flight
+  constexpr int NACC = (SCALE != 0 || SPLIT) ? 1 : 2;    // block scales: one sum of both slots
+  __shared__ __align__(16) float red[kSkWaves][MT][64][4];
+  const int M = g.M, N = g.N, K = g.K;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int n0 = int(blockIdx.x) * kSkN;
+  const int nrows = min(N - n0, kSkN);
+
+  const uint32_t wspan = uint32_t(int64_t(nrows - 1) * g.ldb + K);
+  __amdgpu_buffer_rsrc_t wr[NSL];
+  wr[0] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(g.B0) + int64_t(n0) * g.ldb, 0,
+                                            int(wspan), 0x00020000);
+  if constexpr (!SPLIT)
+    wr[1] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(g.B1) + int64_t(n0) * g.ldb, 0,
+                                              int(wspan), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(g.A), 0, int(uint32_t(int64_t(M - 1) * g.lda + K)), 0x00020000);
+  const uint32_t wv = lr < nrows ? uint32_t(lr) * uint32_t(g.ldb) + uint32_t(lg * 16) : kOob;
+  uint32_t av[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+    av[i] = i * 16 + lr < M ? uint32_t(i * 16 + lr) * uint32_t(g.lda) + uint32_t(lg * 16) : kOob;
+
+  // this wave's steps [s0, s1) of 128 columns
+  const int steps = (K + kSK - 1) / kSK;
+  const int spw = (steps + kSkWaves - 1) / kSkWaves;
+  const int s0 = wave * spw, s1 = min(steps, s0 + spw);
+
+  auto ld = [&](const __amdgpu_buffer_rsrc_t& r, uint32_t voff, int s, int h) -> uint4 {
+    // chunk h * 4 + lg of step s: nothing past K
+    const int k = s * kSK + h * 64;
+    const bool in = s < s1 && k + lg * 16 < K;
+    return __builtin_bit_cast(
+        uint4, __builtin_amdgcn_raw_buffer_load_b128(r, in ? voff : kOob, uint32_t(k), 0));
+  };
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  v4f acc[NACC][MT];
+#pragma unroll
+  for (int a = 0; a < NACC; ++a)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[a][i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+  for (int s = s0; s < s1; s += U) {
+    uint4 w[U][NSL][2], a[U][MT][2];
+    int ew[U][NSL], ea[U][MT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int q = 0; q < NSL; ++q) {
+        w[u][q][0] = ld(wr[q], wv, s + u, 0);
+        w[u][q][1] = ld(wr[q], wv, s + u, 1);
+      }
+      if constexpr (SCALE == 1) {
+        const int k = (s + u) * kSK + lg * 32;
+        const bool in = s + u < s1 && k < K;
+        const uint32_t kb = uint32_t(in ? k >> g.bs_shift : 0);
+#pragma unroll
+        for (int q = 0; q < NSL; ++q)
+          ew[u][q] = in && lr < nrows ? int((q ? g.e_1 : g.e_0)[kb * uint32_t(N) + uint32_t(n0 + lr)]) : 0;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          ea[u][i] = in && i * 16 + lr < M ? int(g.e_a[kb * uint32_t(M) + uint32_t(i * 16 + lr)]) : 0;
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        a[u][i][0] = ld(ar, av[i], s + u, 0);
+        a[u][i][1] = ld(ar, av[i], s + u, 1);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const v8i fa = make_frag(a[u][i][0], a[u][i][1]);
+#pragma unroll
+        for (int q = 0; q < NSL; ++q) {
+          v4f& c = acc[q % NACC][i];
+          const v8i fw = make_frag(w[u][q][0], w[u][q][1]);
+          if constexpr (SCALE == 1)
+            c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                fw, fa, c, BF, AF, 0, int(e8m0_of(ew[u][q])), 0, int(e8m0_of(ea[u][i])));
+          else
+            c = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fw, fa, c, BF, AF, 0, 0, 0, 0);
+        }
+      }
+  }
+
+  // lane l holds columns n0 + 4 * (l / 16) .. + 3 of activation row l % 16
+  float c0s = 1.0f, c1s = 1.0f;
+  if constexpr (SCALE == 0) {
+    const float sa = *g.s_a;
+    c0s = sa * *g.s_0;
+    c1s = SPLIT ? c0s : sa * *g.s_1;
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (SCALE == 1) v[r] = acc[0][i][r];
+      else if constexpr (SPLIT) v[r] = acc[0][i][r] * c0s;
+      else v[r] = acc[0][i][r] * c0s + acc[NACC - 1][i][r] * c1s;
+    }
+    *reinterpret_cast<float4*>(red[wave][i][lane]) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+  __syncthreads();
+  OutT* __restrict__ out = static_cast<OutT*>(g.out);
+#pragma unroll
+  for (int e = threadIdx.x; e < MT * 256; e += kSkWaves * 64) {
+    const int m = e >> 4, c = e & 15;
+    const int sl = (c >> 2) * 16 + (m & 15);
+    float t = red[0][m >> 4][sl][c & 3];
+#pragma unroll
+    for (int w = 1; w < kSkWaves; ++w) t += red[w][m >> 4][sl][c & 3];
+    if (m < M && c < nrows) {
+      if (g.bias) t += g.bias[n0 + c];
+      if constexpr (std::is_same<OutT, float>::value) out[int64_t(m) * g.ldo + n0 + c] = t;
+      else out[int64_t(m) * g.ldo + n0 + c] = f32_to_bf16_rne(t);
+    }
+  }
+}
+
 // Largest byte span any DMA descriptor may cover (offsets are 32-bit and
 // the out-of-range sentinel must stay beyond every span).
 constexpr int64_t kMaxSpan = (int64_t(1) << 31) - (int64_t(1) << 20);
@@ -2126,9 +2281,42 @@ bool exps_al16(const GemmArgs& ga) {
   return al16(ga.e_a) && al16(ga.e_0) && (ga.e_1 == nullptr || al16(ga.e_1));
 }
 
+// The weight stream: few activation rows, whole contraction, descriptors and
+// 32-bit exponent offsets within reach.  Its limit on N is where the 64-column
+// tiles keep enough CUs busy: up to 32 rows 8192 (16 rows: 17.3 against 21.8
+// us at 8192 x 4096, 23.2 against 21.9 at 12288; 32 rows 21.5 against 22.2),
+// up to 64 rows, whose activation tile every workgroup reads again, 2048
+// (6.6 against 7.4 us at 2048 x 1024, level at 2048 x 4096; 15.0 against 13.8
+// at 4096 x 4096).
+bool skinny_eligible(const GemmArgs& ga, bool exps) {
+  if (g_tile_policy != 0 || ga.M > 64 || ga.N > (ga.M <= 32 ? 8192 : 2048)) return false;
+  if (ga.kwrap_b || (ga.kc > 0 && ga.kc < ga.K)) return false;
+  if (int64_t(64) * ga.lda + ga.K >= kMaxSpan || int64_t(kSkN) * ga.ldb + ga.K >= kMaxSpan)
+    return false;
+  // (block exponents: not at the widths that the fused activation-quant GEMM
+  // serves, N <= 512, which give the same bits as that launch)
+  return !exps ||
+         (ga.N > 512 && int64_t(ga.K >> ga.bs_shift) * std::max(ga.M, ga.N) < int64_t(INT32_MAX));
+}
+
+template <int AF, int BF, bool SPLIT, typename OutT, int SCALE>
+int launch_skinny(const GemmArgs& ga, hipStream_t st) {
+  if (ga.bias != nullptr && (reinterpret_cast<uintptr_t>(ga.bias) & 15) != 0) return TCFP_ERR_ALIGN;
+  const unsigned grid = unsigned((ga.N + kSkN - 1) / kSkN);
+  constexpr int T = kSkWaves * 64;
+  if (!grid_x_fits(grid, T)) return TCFP_ERR_SHAPE;
+  if (ga.M <= 16) gemm_skinny_kernel<AF, BF, SPLIT, OutT, SCALE, 1><<<grid, T, 0, st>>>(ga);
+  else if (ga.M <= 32) gemm_skinny_kernel<AF, BF, SPLIT, OutT, SCALE, 2><<<grid, T, 0, st>>>(ga);
+  else gemm_skinny_kernel<AF, BF, SPLIT, OutT, SCALE, 4><<<grid, T, 0, st>>>(ga);
+  return hipGetLastError() == hipSuccess ? TCFP_OK : TCFP_ERR_HIP;
+}
+
 template <int AF, int BF, bool SPLIT, typename OutT, int SCALE>
 int launch_gemm(GemmArgs ga, hipStream_t st) {
   const int m = ga.M, n = ga.N, k = ga.K;
+  // (E4M3 weights: what the quantisers write; other formats keep the tiles)
+  if constexpr (SCALE != 2 && AF != kBF16 && BF == TCFP_FP8_E4M3)
+    if (skinny_eligible(ga, SCALE == 1)) return launch_skinny<AF, BF, SPLIT, OutT, SCALE>(ga, st);
   if constexpr (SCALE == 1 && SPLIT && AF != kBF16 && std::is_same<OutT, float>::value) {
     // block-scaled single GEMM with more full 256 x 128 tiles than CUs: the
     // persistent kernel with the two weight slots on adjacent weight-row

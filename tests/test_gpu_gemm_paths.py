@@ -1,5 +1,5 @@
-"""GEMM paths the dispatcher takes by size: the four-stage small tile with
-block exponents.
+"""GEMM paths the dispatcher takes by size: the weight stream for few
+activation rows, and the four-stage small tile with block exponents.
 
 Bounds: 1e-4 relative Frobenius with fp32 output (the FP8 MFMA's internal sum
 of a block is a flat ~1.5e-5 off a float64 matmul of the same operands; an
@@ -12,6 +12,8 @@ import torch
 from tcfp_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
+
+E4M3, E5M2 = torch.float8_e4m3fn, torch.float8_e5m2
 
 
 def _kernel_names(fn):
@@ -29,6 +31,69 @@ def _rel(out, ref):
 
 def _deq(q, e, bs):
     return q.double() * torch.exp2(e.t().double()).repeat_interleave(bs, dim=1)
+
+
+# rows at the edges of the 16 / 32 / 64-row variants, columns at those of the
+# 16-column workgroups and of the rule (N <= 8192 up to 32 rows, else 2048),
+# contractions with a partial last 128-column step (K % 16 == 0), fewer steps
+# than waves, and steps that the eight waves share unevenly
+FEW = [(1, 16, 16), (1, 1024, 1024), (16, 8192, 4096), (17, 130, 1040), (32, 8192, 272),
+       (33, 2048, 80), (48, 1001, 4096), (64, 2048, 1168), (64, 513, 128)]
+
+
+@pytest.mark.parametrize("dual", [True, False])
+@pytest.mark.parametrize("fmt", [E4M3, E5M2])
+@pytest.mark.parametrize("m,n,k", FEW)
+def test_few_rows_per_tensor(dev, m, n, k, fmt, dual):
+    g = torch.Generator().manual_seed(m * 7 + n + k)
+    a, sa = K.quantize_per_tensor(torch.randn(m, k, generator=g).to(dev), fmt)
+    hi, lo, ih, il = K.dual_quantize_per_tensor(torch.randn(n, k, generator=g).to(dev))
+    bias = torch.randn(n, generator=g).to(dev)
+    ref = (a.double() * sa.double()) @ (
+        hi.double() * ih.double() + (lo.double() * il.double() if dual else 0)).t() + bias.double()
+    for od, tol in ((torch.float32, 1e-4), (torch.bfloat16, 3e-3)):
+        def run():
+            if dual:
+                return K.fused_dual_gemm_forward(a, hi, lo, sa, ih, il, bias=bias, out_dtype=od)
+            return K.fp8_gemm_nt(a, hi, sa, ih, bias=bias, out_dtype=od)
+
+        out = run()
+        assert any("gemm_skinny" in x for x in _kernel_names(run))
+        err = _rel(out, ref)
+        print(f"few rows {m}x{n}x{k} {od} dual={dual} rel_fro {err:.2e}")
+        assert err < tol
+        assert torch.equal(out, run())  # the waves' sums meet in a fixed order
+
+
+@pytest.mark.parametrize("bs", [32, 64, 128])
+@pytest.mark.parametrize("dual", [True, False])
+@pytest.mark.parametrize("m,n,kb", [(1, 1024, 1), (16, 8192, 9), (17, 520, 5), (33, 1001, 17),
+                                    (64, 2048, 32)])
+def test_few_rows_block_exponents(dev, m, n, kb, bs, dual):
+    """Per-column scales spread over many binades, so that an exponent taken
+    from another block or row is an error of order 1."""
+    k = kb * bs
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g) * torch.exp2(torch.randint(-6, 7, (m, k), generator=g))
+    w = torch.randn(n, k, generator=g) * torch.exp2(torch.randint(-6, 7, (n, k), generator=g))
+    a, ea = K.block_quantize_fp8(x.to(dev), bs)
+    hi, lo, eh, el = K.fused_dual_quantize_fp8(w.to(dev), bs)
+    ref = _deq(hi, eh, bs)
+    if dual:
+        ref = ref + _deq(lo, torch.where(el == -128, torch.full_like(el, -127), el), bs)
+    ref = _deq(a, ea, bs) @ ref.t()
+    for od, tol in ((torch.float32, 1e-4), (torch.bfloat16, 3e-3)):
+        def run():
+            if dual:
+                return K.fused_block_scaled_dual_gemm_forward(a, hi, lo, ea, eh, el, bs,
+                                                              out_dtype=od)
+            return K.block_scaled_gemm(a, hi, ea, eh, bs, out_dtype=od)
+
+        out = run()
+        assert any("gemm_skinny" in x for x in _kernel_names(run))
+        err = _rel(out, ref)
+        print(f"few rows {m}x{n}x{k} bs {bs} {od} dual={dual} rel_fro {err:.2e}")
+        assert err < tol
 
 
 @pytest.mark.parametrize("bs", [32, 64, 128])
