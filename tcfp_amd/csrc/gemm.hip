@@ -276,11 +276,16 @@ struct GemmArgs {
 // AQ (SCALE 1 dual, 128 x 64 tile): 0 = A is FP8 codes with exponents e_a;
 // 1 / 2 = A is the bf16 / fp32 activation, block-quantised to E4M3 inside
 // the kernel (the reference's fused activation-quant GEMM).
+// With NS == 3 and SCALE 1, F32BS is the log2 of the smallest block size
+// served (5 or 6): a stage keeps the exponents of 128 >> F32BS K blocks.
 template <int AF, int BF, bool SPLIT, typename OutT, int NW, int BM, int BN, int SCALE, int NS,
           int F32BS = 0, int AQ = 0>
 __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1)) void gemm_nt_dma_kernel(
     GemmArgs g) {
-  static_assert((SCALE == 2 || AQ != 0) == (F32BS != 0), "fp32 block scales and AQ fix the block size");
+  static_assert((SCALE == 2 || AQ != 0 || (SCALE == 1 && NS == 3)) == (F32BS != 0),
+                "fp32 block scales and AQ fix the block size");
+  // K blocks whose exponents a stage of the deep pipelines keeps in LDS
+  constexpr int EXB = SCALE != 1 || NS == 2 ? 0 : F32BS ? kSK >> F32BS : kSK / 32;
   // AQ: bf16 activations on the 128 x 64 tile; fp32 ones (twice the bytes
   // per stage in registers) on a 64 x 64 tile
   static_assert(AQ == 0 || (SCALE == 1 && !SPLIT && AF == 0 && NS == 2 && NW == 4 && BN == 64 &&
@@ -299,9 +304,14 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // rows themselves and DMA only the weight rows)
   constexpr int RPW = (AQ ? 2 * BN : SROWS) / NW;
   constexpr int DI = RPW / 8;       // 1 KiB DMA instructions per wave and stage
-  static_assert(RPW % 16 == 0 && BM % RPW == 0 && BN % RPW == 0, "DMA rows must tile regions");
+  // the 128 x 128 tile (three stages): the waves take 8-row groups of every
+  // region in turn instead of runs of rows inside one region
+  constexpr bool kMid = NW == 4 && BM == 128 && BN == 128 && NS == 3;
+  static_assert(kMid || (RPW % 16 == 0 && BM % RPW == 0 && BN % RPW == 0),
+                "DMA rows must tile regions");
   static_assert(MB >= 1 && NB >= 1, "tile too small for the wave grid");
-  static_assert(NS == 2 || (NS == 4 && (SCALE == 0 || (SCALE == 1 && AQ == 0 && NW == 4))),
+  static_assert(NS == 2 || ((NS == 4 || kMid) &&
+                            (SCALE == 0 || (SCALE == 1 && AQ == 0 && NW == 4))),
                 "deep pipelines: per-tensor scales, or block exponents on four waves");
   static_assert(SCALE != 2 || (NW == 4 && BM == 128 && BN == 64 && NS == 2),
                 "fp32 block scales use the 128 x 64 tile");
@@ -315,15 +325,23 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // block exponents of the deep pipeline: one byte per (32-column K block,
   // stage row) of each buffered stage, brought in with the stage's operands.
   // The byte loads below write one 32-bit LDS word per lane.
-  constexpr bool kExLds = SCALE == 1 && NS == 4;
-  constexpr int kExRows = BM + 2 * BN;               // 64 rows per wave
-  constexpr int kExStage = kExLds ? (kSK / 32) * kExRows * 4 : 0;
-  constexpr int EI = kExLds ? kSK / 32 : 0;          // byte loads per wave and stage
-  static_assert(!kExLds || (kExRows == NW * 64 && BM % 64 == 0 && BN == 64),
-                "each wave brings in 64 rows' exponents");
+  constexpr bool kExLds = EXB != 0;
+  static_assert(kExLds == (SCALE == 1 && NS != 2), "exponents through LDS: the deep pipelines");
+  constexpr int kExRows = BM + 2 * BN;
+  constexpr int kExStage = EXB * kExRows * 4;
+  constexpr int kExG = kExRows / 64;                 // 64-row groups: one byte load each and block
+  constexpr int EI = EXB * kExG / NW;                // byte loads per wave and stage
+  // distinct 64-row groups per wave: load j serves the group of load j % kExP
+  constexpr int kExP = kExLds ? (kMid ? 3 : 1) : 0;
+  static_assert(!kExLds || (kMid ? EI % 3 == 0 : kExG == NW), "exponent groups per wave");
+  // buffered stages of exponents.  Four blocks a stage leave room for two
+  // beside the 128 x 128 tile's operands: those of stage t + 2 are loaded in
+  // stage t, ahead of the operands of stage t + 3
+  constexpr int kExNs = (kMid && EXB == 4) ? 2 : NS;
+  constexpr bool kExEarly = kExNs != NS;
   // AQ: per-wave scratch of one float per (row, block) segment of a stage
   constexpr int kAqS = AQ ? NW * (BM / NW) * (kSK >> F32BS) * 4 : 0;
-  __shared__ __align__(16) uint8_t lds[NS * STAGE + 3 * kScB + kExB + kAqS + NS * kExStage];
+  __shared__ __align__(16) uint8_t lds[NS * STAGE + 3 * kScB + kExB + kAqS + kExNs * kExStage];
 
   const int M = g.M, N = g.N;
   int K = g.K;
@@ -345,7 +363,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // A panels (8 wide groups re-read a large A once per 4 column tiles: the
   // 16384 x 4096 x 16384 split-bf16 wgrad ran 1.80 ms grouped by 8 against
   // 1.69 ms by 4; C3 and C4 shapes measured the same either way)
-  constexpr int G = 4;
+  constexpr int G = kMid ? 8 : 4;
   const int per_group = G * g.tiles_n;
   const int first_m = (l / per_group) * G;
   const int gm = min(g.tiles_m - first_m, G);
@@ -363,11 +381,13 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
 
   // ---- this wave's DMA source: its RPW stage rows lie in the activation,
   // slot-0 or slot-1 region
-  const int srow0 = (AQ ? BM : 0) + wave * RPW;
-  const uint8_t* src;
-  int64_t ld;
-  int rows_left, row_base;
-  if (srow0 < BM) {
+  const int srow0 = (AQ ? BM : 0) + (kMid ? wave * 8 : wave * RPW);
+  const uint8_t* src = g.A;
+  int64_t ld = 0;
+  int rows_left = 0, row_base = 0;
+  if constexpr (kMid) {
+    // (per region below)
+  } else if (srow0 < BM) {
     src = g.A + koff + int64_t(m0) * g.lda; ld = g.lda; rows_left = min(M - m0, BM); row_base = srow0;
   } else if (srow0 < BM + BN) {
     src = g.B0 + (g.kwrap_b ? 0 : koff) + int64_t(n0) * g.ldb; ld = g.ldb;
@@ -377,22 +397,51 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
     rows_left = min(N - n1, BN); row_base = srow0 - BM - BN;
   }
   // a wrapping B region addresses contraction bytes koff + t * kSK modulo kwrap_b
-  const uint32_t kwrap = srow0 >= BM ? uint32_t(g.kwrap_b) : 0u;
+  const uint32_t kwrap = !kMid && srow0 >= BM ? uint32_t(g.kwrap_b) : 0u;
   const uint32_t nrec =
       rows_left > 0 ? uint32_t(int64_t(rows_left - 1) * ld + (kwrap ? int(kwrap) : K)) : 0u;
   const v4i rsrc = make_rsrc(src, nrec);
   // Instruction i fills stage rows srow0 + i*8 .. +8 (1 KiB); lane writes row
   // +lane/8 at physical chunk lane%8.  srow0 is a multiple of 16, so the
   // logical chunk depends on i only through i's low bit.
-  const int chunk0 = (lane & 7) ^ swz(lane >> 3);        // even i
-  const int chunk1 = (lane & 7) ^ swz(8 + (lane >> 3));  // odd i
+  // (kMid: instruction i fills rows (i % 4) * 32 + wave * 8 .. + 8 of region
+  // i / 4: the chunk depends on the wave alone.)
+  const int chunk0 = (lane & 7) ^ swz((kMid ? wave * 8 : 0) + (lane >> 3));             // even i
+  const int chunk1 = kMid ? chunk0 : (lane & 7) ^ swz(8 + (lane >> 3));  // odd i
   uint32_t voff[DI];
+  v4i rsrc3[kMid ? 3 : 1];
+  if constexpr (kMid) {
 #pragma unroll
-  for (int i = 0; i < DI; ++i) {
-    const int r = row_base + i * 8 + (lane >> 3);
-    const int c = (i & 1) ? chunk1 : chunk0;
-    voff[i] = r < rows_left ? uint32_t(int64_t(r) * ld + c * 16) : kOob;
+    for (int q = 0; q < 3; ++q) {
+      const int64_t l3 = q == 0 ? g.lda : g.ldb;
+      const int left = q == 0 ? min(M - m0, BM) : min(N - (q == 1 ? n0 : n1), BN);
+      const uint8_t* b3 = q == 0 ? g.A + koff + int64_t(m0) * g.lda
+                                 : (q == 1 ? g.B0 : g.B1) + koff + int64_t(q == 1 ? n0 : n1) * g.ldb;
+      rsrc3[q] = make_rsrc(b3, left > 0 ? uint32_t(int64_t(left - 1) * l3 + K) : 0u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = i * 32 + srow0 + (lane >> 3);
+        voff[4 * q + i] = r < left ? uint32_t(int64_t(r) * l3 + chunk0 * 16) : kOob;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < DI; ++i) {
+      const int r = row_base + i * 8 + (lane >> 3);
+      const int c = (i & 1) ? chunk1 : chunk0;
+      voff[i] = r < rows_left ? uint32_t(int64_t(r) * ld + c * 16) : kOob;
+    }
   }
+  // LDS offset of instruction i from the wave's base, and its descriptor
+  auto dma_dst = [](int i) -> uint32_t {
+    return kMid ? uint32_t(((i / 4) * 128 + (i % 4) * 32) * kRowB) : uint32_t(i) * 1024u;
+  };
+  auto dma_op = [&](int i, uint32_t vo, uint32_t soff, uint32_t dst) {
+    if constexpr (kMid) dma16(rsrc3[i / 4], vo, soff, dst + dma_dst(i));
+    else dma16(rsrc, vo, soff, dst + dma_dst(i));
+  };
+  // buffer of stage t
+  auto buf = [](int t) -> int { return NS == 3 ? t % 3 : t & (NS - 1); };
   const uint32_t lds_base =
       uint32_t(reinterpret_cast<uintptr_t>((TCFP_LDS uint8_t*)lds)) + uint32_t(srow0) * kRowB;
   const int nt = (K + kSK - 1) / kSK;
@@ -426,34 +475,42 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // stage rows 64 w .. + 63 (one array, one row per lane; rows past the
   // matrix read 0), K block by K block.  Byte loads: an exponent array's
   // rows start at any alignment (M, N are any numbers).
-  v4i exrsrc = {};
-  uint32_t exvoff = kOob, exlds = 0;
-  int exld = 0;
+  v4i exrsrc[kExLds ? kExP : 1] = {};
+  uint32_t exvoff[kExLds ? kExP : 1] = {}, exdst[kExLds ? kExP : 1] = {};
+  int exld[kExLds ? kExP : 1] = {}, exb[kExLds ? kExP : 1] = {};
   if constexpr (kExLds) {
-    const int er = wave * 64;
-    const int8_t* eb;
-    int base, rows;
-    if (er < BM) {
-      eb = g.e_a; base = m0 + er; rows = M;
-    } else if (er < BM + BN) {
-      eb = g.e_0; base = n0; rows = N;
-    } else {
-      eb = SPLIT ? g.e_0 : g.e_1; base = n1; rows = N;
+#pragma unroll
+    for (int j = 0; j < kExP; ++j) {
+      const int x = NW * j + wave;             // load x of the stage: group x % kExG, block x / kExG
+      const int er = (x % kExG) * 64;
+      exb[j] = x / kExG;
+      const int8_t* eb;
+      int base, rows;
+      if (er < BM) {
+        eb = g.e_a; base = m0 + er; rows = M;
+      } else if (er < BM + BN) {
+        eb = g.e_0; base = n0 + er - BM; rows = N;
+      } else {
+        eb = SPLIT ? g.e_0 : g.e_1; base = n1 + er - BM - BN; rows = N;
+      }
+      exld[j] = rows;
+      exrsrc[j] = make_rsrc(eb, uint32_t(int64_t(K >> g.bs_shift) * rows));
+      exvoff[j] = base + lane < rows ? uint32_t(base + lane) : kOob;
+      exdst[j] = uint32_t(reinterpret_cast<uintptr_t>((TCFP_LDS uint8_t*)lds)) +
+                 uint32_t(NS * STAGE) + uint32_t(er) * 4;
     }
-    exld = rows;
-    exrsrc = make_rsrc(eb, uint32_t(int64_t(K >> g.bs_shift) * rows));
-    exvoff = base + lane < rows ? uint32_t(base + lane) : kOob;
-    exlds = uint32_t(reinterpret_cast<uintptr_t>((TCFP_LDS uint8_t*)lds)) +
-            uint32_t(NS * STAGE) + uint32_t(er) * 4;
   }
-  // K block b (32 columns) of stage t -> the stage's exponent slots
-  auto issue_ex = [&](int t, int b) {
+  // byte load j of stage t: 64 rows of one K block -> the stage's exponent slots
+  auto issue_ex = [&](int t, int j) {
     if constexpr (kExLds) {
-      const int k = t * kSK + b * 32;
+      const int p = j % kExP;
+      const int b = exb[p] + (j / kExP) * (NW * kExP / kExG);
+      const int k = t * kSK + b * (kSK / EXB);
       const bool in = k < K;
-      const uint32_t soff = uint32_t(in ? k >> g.bs_shift : 0) * uint32_t(exld);
-      dma1(exrsrc, in ? exvoff : kOob, soff,
-           exlds + uint32_t(t & (NS - 1)) * kExStage + uint32_t(b * kExRows * 4));
+      const uint32_t soff = uint32_t(in ? k >> g.bs_shift : 0) * uint32_t(exld[p]);
+      const int eb = kExNs == 3 ? t % 3 : t & (kExNs - 1);
+      dma1(exrsrc[p], in ? exvoff[p] : kOob, soff,
+           exdst[p] + uint32_t(eb) * kExStage + uint32_t(b * kExRows * 4));
     }
   };
 
@@ -461,7 +518,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // end are issued as all-out-of-range loads (zeros into a buffer nobody
   // reads again), so the issue stays branch-free.
   auto issue = [&](int t) {
-    const uint32_t dst = lds_base + uint32_t(t & (NS - 1)) * STAGE;
+    const uint32_t dst = lds_base + uint32_t(buf(t)) * STAGE;
     const bool live = t < nt;
     uint32_t soff = uint32_t(live ? t : 0) * kSK;
     if (kwrap) {
@@ -469,13 +526,15 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
       if (soff >= kwrap) soff -= kwrap;
     }
     const bool last = t == nt - 1;
+    if (t < kExNs) {
+#pragma unroll
+      for (int j = 0; j < EI; ++j) issue_ex(t, j);
+    }
 #pragma unroll
     for (int i = 0; i < DI; ++i) {
       const int c = (i & 1) ? chunk1 : chunk0;
-      dma16(rsrc, (!live || (last && c * 16 >= krem)) ? kOob : voff[i], soff, dst + i * 1024);
+      dma_op(i, (!live || (last && c * 16 >= krem)) ? kOob : voff[i], soff, dst);
     }
-#pragma unroll
-    for (int b = 0; b < EI; ++b) issue_ex(t, b);
     if constexpr (SCALE == 2) {
       if (live && wave < (kSK >> f32_bsh)) {
         const int kb = min(((t * kSK) >> f32_bsh) + wave, nkb - 1);
@@ -722,8 +781,9 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   auto ex_code = [&](int t, int h, int x) -> uint32_t {
     const int row = x < NF ? BM + (x / NB) * BN + wn * TNW + (x % NB) * 32 + lr
                            : wm * TMW + (x - NF) * 32 + lr;
+    const int eb = kExNs == 3 ? t % 3 : t & (kExNs - 1);
     const uint32_t u = *reinterpret_cast<const uint32_t*>(
-        lds + NS * STAGE + (t & (NS - 1)) * kExStage + ((2 * h + lg) * kExRows + row) * 4);
+        lds + NS * STAGE + eb * kExStage + ((EXB == 4 ? 2 * h + lg : h) * kExRows + row) * 4);
     const uint32_t v = u ^ 128u;
     return (v > 1u ? v : 1u) - 1u;
   };
@@ -746,7 +806,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // Fragments of sub-step h of stage t: [0, NF) weights (slot, n-block),
   // [NF, NF + MB) activations (m-block).
   auto read_frags = [&](v8i* f, int t, int h) {
-    const uint8_t* st = lds + (t & (NS - 1)) * STAGE;
+    const uint8_t* st = lds + buf(t) * STAGE;
 #pragma unroll
     for (int q = 0; q < NF; ++q) {
       const int rb = (BM + (q / NB) * BN + wn * TNW + (q % NB) * 32) * kRowB;
@@ -827,9 +887,10 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // touch no memory, so without it they drift past the barrier and the LDS
   // reads before it are left with nothing to hide behind.
   // With NS stages, the DMAs of stages t+2 .. t+NS-1 may stay in flight.
-  constexpr int kInflight = (NS - 2) * (DI + EI);
-  // four stages in flight on one four-wave workgroup per CU
-  constexpr bool kDeep = NW == 4 && NS == 4 && SCALE != 2 && AQ == 0;
+  // (kExEarly: of stage t + 2 only the operands)
+  constexpr int kInflight = kExEarly ? DI : (NS - 2) * (DI + EI);
+  // three or four stages in flight on one four-wave workgroup per CU
+  constexpr bool kDeep = NW == 4 && NS > 2 && SCALE != 2 && AQ == 0;
   auto sync_all = [&]() {
     __builtin_amdgcn_sched_barrier(0);
     // vmcnt(kInflight) lgkmcnt(0), expcnt untouched
@@ -859,7 +920,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
       // (the exponent loads were issued before all of them and are complete;
       // a wave that also loads fp32 scales issues one more per stage, which
       // only makes this wait longer)
-      constexpr int kPro = (NS - 1) * (DI + EI);
+      constexpr int kPro = (NS - 1) * DI + (kExNs - 1) * EI;
       __builtin_amdgcn_s_waitcnt((kPro & 15) | (7 << 4) | ((kPro >> 4) << 14));
     }
     __builtin_amdgcn_s_barrier();
@@ -1001,9 +1062,10 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
     constexpr int NFR = NF + MB;  // fragments per sub-step
     constexpr int NP = NF * MB;   // (fragment, m-block) pairs per sub-step
     constexpr int SL = 2 * NP;    // MFMA pairs (slots) per stage
-    constexpr int DSL = 6;        // slots after the barrier that carry the DMA
-    constexpr int RSL = 5;        // slots after the barrier that carry the reads
-    static_assert(1 + DSL <= SL && 1 + RSL < SL, "deep schedule slots");
+    constexpr int ESL = kMid && kExLds ? 3 : 0;  // slots after the barrier with the exponent loads,
+    constexpr int DSL = kMid ? (kExLds ? 6 : 12) : 6;  // then those with the operand DMA
+    constexpr int RSL = kMid ? 12 : 5;  // slots after the barrier that carry the reads
+    static_assert(1 + ESL + DSL <= SL && 1 + RSL < SL, "deep schedule slots");
     v8i g0[NFR], g1[NFR];
     uint32_t sg[2 * NFR];  // the other stage's E8M0 codes (block exponents)
     // chunks past K in the last stage (per lane, even / odd DMA instruction)
@@ -1017,7 +1079,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
       // fragment r of stage t + 1 (sub-step r / NFR)
       auto rd = [&](int r) {
         const int h = r / NFR, x = r % NFR;
-        const uint8_t* st = lds + ((t + 1) & (NS - 1)) * STAGE;
+        const uint8_t* st = lds + buf(t + 1) * STAGE;
         const int rb = x < NF ? (BM + (x / NB) * BN + wn * TNW + (x % NB) * 32) * kRowB
                               : (wm * TMW + (x - NF) * 32) * kRowB;
         (h ? x1 : x0)[x] = make_frag(lds_read16(st, rb + ro[h][0]), lds_read16(st, rb + ro[h][1]));
@@ -1033,7 +1095,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
         soff += uint32_t(koff);
         if (soff >= kwrap) soff -= kwrap;
       }
-      uint32_t dst = lds_base + uint32_t(tr & (NS - 1)) * STAGE;
+      uint32_t dst = lds_base + uint32_t(buf(tr)) * STAGE;
       uint32_t vo[DI];
 #pragma unroll
       for (int i = 0; i < DI; ++i) {
@@ -1048,12 +1110,20 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
         mf(s);
         __builtin_amdgcn_sched_barrier(0);
         const int j = s - 1;
-        if (j < DSL) {
+        if constexpr (ESL > 0) {
+          if (j < ESL) {
 #pragma unroll
-          for (int i = j * DI / DSL; i < (j + 1) * DI / DSL; ++i)
-            dma16(rsrc, vo[i], soff, dst + i * 1024);
+            for (int x = j * EI / ESL; x < (j + 1) * EI / ESL; ++x) issue_ex(t + kExNs, x);
+          }
+        }
+        if (j >= ESL && j < ESL + DSL) {
+          const int d = j - ESL;
 #pragma unroll
-          for (int b = j * EI / DSL; b < (j + 1) * EI / DSL; ++b) issue_ex(tr, b);
+          for (int i = d * DI / DSL; i < (d + 1) * DI / DSL; ++i) dma_op(i, vo[i], soff, dst);
+          if constexpr (ESL == 0) {
+#pragma unroll
+            for (int x = d * EI / DSL; x < (d + 1) * EI / DSL; ++x) issue_ex(tr, x);
+          }
         }
         if (j < RSL) {
 #pragma unroll
@@ -2233,6 +2303,7 @@ constexpr int64_t kMaxSpan = (int64_t(1) << 31) - (int64_t(1) << 20);
 // 3 = 128 x 64 with eight waves in the one-round deep-pipeline case,
 // 4 = 256 x 128 with one workgroup per tile (no persistent launch),
 // 5 = the four-wave persistent 256 x 128 tile (per-tensor dual, bf16 out).
+// 6 = 128 x 128 per slot with four waves and three stages.
 int g_tile_policy = 0;
 
 int num_cus() {
@@ -2311,6 +2382,60 @@ int launch_skinny(const GemmArgs& ga, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? TCFP_OK : TCFP_ERR_HIP;
 }
 
+// The 128 x 128 tile of the dual GEMM: between the small tile's one round
+// (deep) and the large tile's.  A 128 x 64 tile pair per CU moves 64 KiB into
+// LDS per 1024 cycles of MFMA, the L2 -> LDS limit, and its two-stage loop
+// waits on it (block exponents, in registers, add a drain per stage); this
+// tile moves 48 KiB and keeps two stages in flight.  M x N x K, before ->
+// after: per tensor 1000 x 4096 x 4096 38.4 -> 33.2 us, 2048 x 2048 x 4096
+// 36.5 -> 31.7, 1000 x 2560 x 2048 16.9 -> 15.4; block 64 1000 x 4096 x 4096
+// 61.9 -> 36.0, 2048 x 2048 x 4096 49.4 -> 35.2, 600 x 4096 x 2048 26.1 -> 18.2.
+// Its loop runs at the power-capped matrix rate (a 1024-column step of K
+// 6.4 us at 1000 x 4096); launch, first loads and output are ~7 us beside it.
+// Where the line lies: shorter contractions in more than one round lose the
+// overlap of two workgroups' epilogues (per tensor 1100 x 4096 x 4096 55.6 ->
+// 52.0, x 1024 19.2 -> 21.0; 1300 x 4096 x 2048 29.8 -> 30.3; one round, K 1024,
+// 13.5 -> 13.2, K 512 10.7 -> 10.9; block 64 2048 x 2048 x 512 12.2 -> 10.7, x 256
+// level, 1500 x 4096 x 512 18.4 -> 18.9, 520 x 8192 x 1024 27.1 -> 23.0).
+// From one large tile per CU on the large tile is faster (2048 x 4096 x 2048
+// 33.9 against 36.9), and so is the small tile's one round (512 x 4096 x 4096
+// 23.5 against 30.6).  Single products and bf16 operands measured level: not
+// built.
+bool mid_eligible(const GemmArgs& ga, bool exps) {
+  if (g_tile_policy != 0 && g_tile_policy != 6) return false;
+  if (ga.kwrap_b || (ga.kc > 0 && ga.kc < ga.K)) return false;
+  if (int64_t(128) * ga.lda + ga.K >= kMaxSpan || int64_t(128) * ga.ldb + ga.K >= kMaxSpan)
+    return false;
+  if (exps && int64_t(ga.K >> ga.bs_shift) * std::max(ga.M, ga.N) >= kMaxSpan) return false;
+  if (g_tile_policy == 6) return true;
+  const auto tiles = [&](int bm, int bn) {
+    return int64_t((ga.M + bm - 1) / bm) * ((ga.N + bn - 1) / bn);
+  };
+  const int64_t cus = num_cus();
+  if (tiles(256, 128) >= cus || tiles(128, 64) <= cus) return false;
+  const bool one_round = tiles(128, 128) <= cus;
+  return exps ? ga.K >= (one_round ? 512 : 1024) : ga.K >= (one_round ? 1024 : 3072);
+}
+
+template <int AF, int BF, typename OutT, int SCALE>
+int launch_mid(GemmArgs ga, hipStream_t st) {
+  ga.tiles_m = (ga.M + 127) / 128;
+  ga.tiles_n = (ga.N + 127) / 128;
+  if (ga.bias != nullptr && (reinterpret_cast<uintptr_t>(ga.bias) & 15) != 0) return TCFP_ERR_ALIGN;
+  const int64_t tiles = int64_t(ga.tiles_m) * ga.tiles_n;
+  if (!grid_x_fits(tiles, 256)) return TCFP_ERR_SHAPE;
+  const unsigned grid = unsigned(tiles);
+  if constexpr (SCALE == 1) {
+    if (ga.bs_shift == 5)
+      gemm_nt_dma_kernel<AF, BF, false, OutT, 4, 128, 128, 1, 3, 5><<<grid, 256, 0, st>>>(ga);
+    else
+      gemm_nt_dma_kernel<AF, BF, false, OutT, 4, 128, 128, 1, 3, 6><<<grid, 256, 0, st>>>(ga);
+  } else {
+    gemm_nt_dma_kernel<AF, BF, false, OutT, 4, 128, 128, SCALE, 3><<<grid, 256, 0, st>>>(ga);
+  }
+  return hipGetLastError() == hipSuccess ? TCFP_OK : TCFP_ERR_HIP;
+}
+
 template <int AF, int BF, bool SPLIT, typename OutT, int SCALE>
 int launch_gemm(GemmArgs ga, hipStream_t st) {
   const int m = ga.M, n = ga.N, k = ga.K;
@@ -2346,6 +2471,8 @@ int launch_gemm(GemmArgs ga, hipStream_t st) {
       return hipGetLastError() == hipSuccess ? TCFP_OK : TCFP_ERR_HIP;
     }
   }
+  if constexpr (SCALE != 2 && !SPLIT && AF != kBF16)
+    if (mid_eligible(ga, SCALE == 1)) return launch_mid<AF, BF, OutT, SCALE>(ga, st);
   // large tile unless it would leave CUs idle
   const int big_tiles = ((m + 255) / 256) * ((n + (SPLIT ? 255 : 127)) / (SPLIT ? 256 : 128));
   // (block-scaled single GEMMs keep two accumulator sets, which only the
@@ -2754,7 +2881,7 @@ extern "C" int tcfp_wtquant_block_dual_gemm(const uint8_t* a, int a_fmt, int64_t
 }
 
 extern "C" int tcfp_gemm_set_tile_policy(int policy) {
-  if (policy < 0 || policy > 5) return TCFP_ERR_SHAPE;
+  if (policy < 0 || policy > 6) return TCFP_ERR_SHAPE;
   g_tile_policy = policy;
   return TCFP_OK;
 }

@@ -119,3 +119,50 @@ def test_four_stage_block_exponents_match_two_stage(dev, m, n, k, bs):
     assert _rel(out, ref) < 1e-4
     single = K.block_scaled_gemm(a, hi, ea, eh, bs)
     assert _rel(single, _deq(a, ea, bs) @ _deq(hi, eh, bs).t()) < 1e-4
+
+
+# the 128 x 128 tile: full and partial tiles on both sides, a partial last
+# stage (K % 128 != 0), fewer stages than buffers under the forcing policy,
+# and the shapes the rule sends there
+MID = [("auto", 1000, 4096, 1040, 0), ("auto", 2048, 2048, 1024, 64), ("auto", 600, 4000, 2048, 32),
+       ("auto", 600, 4000, 2048, 128), ("mid", 130, 200, 16, 0), ("mid", 1, 129, 272, 0),
+       ("mid", 257, 250, 64, 64), ("mid", 100, 385, 96, 32), ("mid", 128, 128, 384, 128)]
+
+
+@pytest.mark.parametrize("od", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("policy,m,n,k,bs", MID)
+def test_mid_tile_matches_small_tile(dev, policy, m, n, k, bs, od):
+    """The 128 x 128 tile's bits are the 128 x 64 tile's (the same products in
+    the same order of K), with a bias, and within the bound of float64."""
+    g = torch.Generator().manual_seed(m + n + k + bs)
+    x = torch.randn(m, k, generator=g).to(dev)
+    w = (torch.randn(n, k, generator=g)
+         * torch.exp2(torch.randint(-9, 9, (n, 1), generator=g))).to(dev)
+    bias = torch.randn(n, generator=g).to(dev)
+    if bs:
+        a, ea = K.block_quantize_fp8(x, bs, E5M2)
+        hi, lo, eh, el = K.fused_dual_quantize_fp8(w, bs)
+        ref = _deq(a, ea, bs) @ (_deq(hi, eh, bs) + _deq(lo, el, bs)).t()
+
+        def run():
+            return K.fused_block_scaled_dual_gemm_forward(a, hi, lo, ea, eh, el, bs, bias=bias,
+                                                          out_dtype=od)
+    else:
+        a, sa = K.quantize_per_tensor(x, E5M2)
+        hi, lo, ih, il = K.dual_quantize_per_tensor(w)
+        ref = (a.double() * sa.double()) @ (hi.double() * ih.double()
+                                            + lo.double() * il.double()).t()
+
+        def run():
+            return K.fused_dual_gemm_forward(a, hi, lo, sa, ih, il, bias=bias, out_dtype=od)
+    try:
+        K.set_gemm_tile_policy("small")
+        small = run()
+        K.set_gemm_tile_policy(policy)
+        names = _kernel_names(run)
+        out = run()
+    finally:
+        K.set_gemm_tile_policy("auto")
+    assert any("4, 128, 128, " in s for s in names), names
+    assert torch.equal(out, small)
+    assert _rel(out, ref + bias.double()) < (1e-4 if od == torch.float32 else 3e-3)
