@@ -190,6 +190,26 @@ def lib() -> ctypes.CDLL:
     return _lib if _lib is not None else load_library()
 
 
+_host = None
+
+
+def host():
+    """The native host path (``_tcfp_host``, built with the library): the
+    checks, allocations and C-ABI calls of the ops in the layers' passes."""
+    global _host
+    if _host is None:
+        lib()
+        try:
+            from . import _tcfp_host
+        except ImportError as e:
+            raise RuntimeError(
+                f"tcfp_amd native host module not loadable ({e}); build it with "
+                "`python -m tcfp_amd.build` (or __graft_entry__.build())"
+            ) from e
+        _host = _tcfp_host
+    return _host
+
+
 def is_available() -> bool:
     """True when the library is built and a GPU is visible."""
     if not LIB_PATH.exists():
@@ -244,22 +264,7 @@ def workspace(device: torch.device) -> torch.Tensor:
     return ws
 
 
-_bws: dict[tuple[int, int], torch.Tensor] = {}
-MAX_BATCH_JOBS = 4
-
-
-def batch_workspace(device: torch.device) -> torch.Tensor:
-    """``tcfp_quantize_batch``'s reduction scratch (room for its largest
-    batch) for the current stream of ``device``; stream order makes one per
-    (device, stream) safe."""
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    key = (idx, stream_of(device))
-    ws = _bws.get(key)
-    if ws is None:
-        nbytes = int(lib().tcfp_quantize_batch_workspace_bytes(MAX_BATCH_JOBS))
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        _bws[key] = ws
-    return ws
+MAX_BATCH_JOBS = 4  # tensors per tcfp_quantize_batch
 
 
 def require_gpu(*tensors: torch.Tensor) -> torch.device:

@@ -5,7 +5,9 @@
 Each ``csrc/*.hip`` file is compiled by ``hipcc --offload-arch=gfx950`` to
 an object under ``tcfp_amd/_build/`` and the objects are linked into
 ``tcfp_amd/libtcfp_hip.so``.  The library has no libtorch dependency: the
-Python side binds it through ctypes.
+Python side binds it through ctypes, and through ``tcfp_amd/_tcfp_host.so``
+(``csrc/host.cpp``, host C++ against torch's headers and the library), the
+native host path of the ops that every layer pass makes.
 """
 from __future__ import annotations
 
@@ -13,12 +15,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libtcfp_hip.so"
+HOST = PKG / "_tcfp_host.so"
 INCLUDE = PKG.parent / "include"
 
 ARCH = "gfx950"
@@ -52,6 +56,26 @@ def hipcc() -> str:
     return cand
 
 
+def host_commands(obj: Path, out: Path) -> tuple[list[str], list[str]]:
+    """Compile and link commands of the native host module (no GPU code)."""
+    import torch
+    from torch.utils import cpp_extension as ext
+
+    cxx = shutil.which("g++") or "g++"
+    inc = [*ext.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    compile_ = [
+        cxx, "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        *(f"-I{i}" for i in inc), "-c", str(CSRC / "host.cpp"), "-o", str(obj),
+    ]
+    link = [
+        cxx, "-shared", str(obj), "-o", str(out), *(f"-L{p}" for p in ext.library_paths()),
+        "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-L{PKG}",
+        "-ltcfp_hip", "-Wl,-rpath,$ORIGIN",
+    ]
+    return compile_, link
+
+
 def build(verbose: bool = True) -> Path:
     BUILD.mkdir(exist_ok=True)
     cc = hipcc()
@@ -65,6 +89,12 @@ def build(verbose: bool = True) -> Path:
         if verbose:
             print("[tcfp_amd.build]", " ".join(cmd), flush=True)
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
+    host_tmp = HOST.with_suffix(".so.tmp")
+    host_cc, host_link = host_commands(BUILD / "host.o", host_tmp)
+    if verbose:
+        print("[tcfp_amd.build]", " ".join(host_cc), flush=True)
+    procs.append((CSRC / "host.cpp",
+                  subprocess.Popen(host_cc, stdout=subprocess.PIPE, stderr=subprocess.STDOUT)))
     failed = []
     for src, p in procs:
         out, _ = p.communicate()
@@ -83,6 +113,10 @@ def build(verbose: bool = True) -> Path:
         print("[tcfp_amd.build]", " ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
     os.replace(tmp, LIB)
+    if verbose:
+        print("[tcfp_amd.build]", " ".join(host_link), flush=True)
+    subprocess.run(host_link, check=True)
+    os.replace(host_tmp, HOST)
     return LIB
 
 

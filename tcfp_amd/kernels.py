@@ -96,29 +96,7 @@ def quantize_per_tensor(
     the 2-D view) when ``transpose``, plus the fp32 ``scale`` when
     ``return_scale``.  ``x`` is viewed as ``[numel / x.shape[-1], x.shape[-1]]``.
     """
-    dev = _hip.require_gpu(x, scale)
-    xc = x if x.is_contiguous() else x.contiguous()
-    cols = xc.shape[-1] if xc.dim() > 0 else 1
-    rows = xc.numel() // cols if cols else 0
-    q = torch.empty(x.shape, dtype=fp8_dtype, device=dev)
-    q_t = torch.empty((cols, rows), dtype=fp8_dtype, device=dev) if transpose else None
-    inv = torch.empty(1, dtype=torch.float32, device=dev)
-    scale_out = torch.empty(1, dtype=torch.float32, device=dev) if return_scale else None
-    s_in = _scalar(scale.to(torch.float32), "scale") if scale is not None else None
-    ws = _hip.workspace(dev) if scale is None else None
-    check(
-        _hip.lib().tcfp_quantize_per_tensor(
-            ptr(xc), _in_dtype(xc), rows, cols, _fmt(fp8_dtype), ptr(s_in), ptr(q), ptr(q_t),
-            ptr(scale_out), ptr(inv), ptr(ws), _hip.stream_of(dev),
-        ),
-        "quantize_per_tensor",
-    )
-    out = (q, inv)
-    if transpose:
-        out = out + (q_t,)
-    if return_scale:
-        out = out + (scale_out,)
-    return out
+    return _hip.host().quantize_per_tensor(x, fp8_dtype, scale, transpose, return_scale)
 
 
 def quantize_per_tensor_sr(
@@ -197,28 +175,7 @@ def quantize_per_tensor_colsum(
     codes (``:494``).  Returns ``(q, inv, col_sum)`` or, with ``transpose``,
     ``(q, inv, q_t, col_sum)``.  Needs ``x.shape[-1] % 8 == 0``.
     """
-    dev = _hip.require_gpu(x)
-    xc = x if x.is_contiguous() else x.contiguous()
-    cols = xc.shape[-1]
-    rows = xc.numel() // cols if cols else 0
-    if cols % 8 != 0:
-        raise ValueError(f"column count ({cols}) must be divisible by 8")
-    q = torch.empty(x.shape, dtype=fp8_dtype, device=dev)
-    q_t = torch.empty((cols, rows), dtype=fp8_dtype, device=dev) if transpose else None
-    inv = torch.empty(1, dtype=torch.float32, device=dev)
-    cs = torch.empty(cols, dtype=torch.float32, device=dev)
-    nbytes = int(_hip.lib().tcfp_colsum_workspace_bytes(rows, cols))
-    cws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
-    check(
-        _hip.lib().tcfp_quantize_per_tensor_colsum(
-            ptr(xc), _in_dtype(xc), rows, cols, _fmt(fp8_dtype), ptr(q), ptr(q_t), ptr(inv),
-            ptr(cs), ptr(_hip.workspace(dev)), ptr(cws), nbytes, _hip.stream_of(dev),
-        ),
-        "quantize_per_tensor_colsum",
-    )
-    if transpose:
-        return q, inv, q_t, cs
-    return q, inv, cs
+    return _hip.host().quantize_per_tensor_colsum(x, fp8_dtype, transpose)
 
 
 def gelu_quantize_per_tensor(
@@ -344,6 +301,13 @@ def dual_quantize_per_tensor(
     the amax rule when that std is below 1e-6.  ``stochastic_hi`` (only with
     ``sigma_factor``) rounds the W_hi codes stochastically.
     """
+    if stochastic_hi and sigma_factor is None:
+        raise ValueError("stochastic_hi applies to NF-aware scaling only (pass sigma_factor)")
+    if (stochastic_lo or stochastic_hi) and seed is None:
+        seed = int(torch.randint(0, 2**62, (1,)).item())
+    if sigma_factor is None:
+        return _hip.host().dual_quantize_per_tensor(weight, error_buf, update_ef, stochastic_lo,
+                                                    transposed, seed or 0)
     dev = _hip.require_gpu(weight, error_buf)
     assert weight.dim() == 2, "weight must be 2-D (N, K)"
     w = weight if weight.is_contiguous() else weight.contiguous()
@@ -360,26 +324,9 @@ def dual_quantize_per_tensor(
     inv_lo = torch.empty(1, dtype=torch.float32, device=dev)
     w_hi_t = torch.empty((k, n), dtype=torch.float8_e4m3fn, device=dev) if transposed else None
     w_lo_t = torch.empty((k, n), dtype=torch.float8_e4m3fn, device=dev) if transposed else None
-    if stochastic_hi and sigma_factor is None:
-        raise ValueError("stochastic_hi applies to NF-aware scaling only (pass sigma_factor)")
-    if (stochastic_lo or stochastic_hi) and seed is None:
-        seed = int(torch.randint(0, 2**62, (1,)).item())
-    if sigma_factor is not None:
-        _dual_quantize_nf(
-            w, n, k, error_buf, update_ef, sigma_factor, stochastic_hi, stochastic_lo, seed,
-            None, None, 0.0, False, None, None, w_hi, w_lo, inv_hi, inv_lo, w_hi_t, w_lo_t, dev,
-        )
-        if transposed:
-            return w_hi, w_lo, inv_hi, inv_lo, w_hi_t, w_lo_t
-        return w_hi, w_lo, inv_hi, inv_lo
-    check(
-        _hip.lib().tcfp_dual_quantize_per_tensor(
-            ptr(w), _in_dtype(w), n, k, ptr(error_buf), int(bool(update_ef)),
-            int(bool(stochastic_lo)), int(seed or 0), 0, ptr(w_hi), ptr(w_lo), ptr(inv_hi),
-            ptr(inv_lo), ptr(w_hi_t), ptr(w_lo_t), ptr(_hip.workspace(dev)),
-            _hip.stream_of(dev),
-        ),
-        "dual_quantize_per_tensor",
+    _dual_quantize_nf(
+        w, n, k, error_buf, update_ef, sigma_factor, stochastic_hi, stochastic_lo, seed,
+        None, None, 0.0, False, None, None, w_hi, w_lo, inv_hi, inv_lo, w_hi_t, w_lo_t, dev,
     )
     if transposed:
         return w_hi, w_lo, inv_hi, inv_lo, w_hi_t, w_lo_t
@@ -406,39 +353,7 @@ def quantize_batch(dual=(), act=()):
     if not fits:
         return ([dual_quantize_per_tensor(w, e, u, transposed=t) for w, e, u, t in dual],
                 [quantize_per_tensor(x, f, transpose=t) for x, f, t in act])
-    dev = _hip.require_gpu(*[t for w, e, _, _ in dual for t in (w, e)],
-                           *[x for x, _, _ in act])
-    jobs = (_hip.QuantJob * (len(dual) + len(act)))()
-    res_d, res_a = [], []
-    for i, (w, e, u, t) in enumerate(dual):
-        w = w if w.is_contiguous() else w.contiguous()
-        n, k = w.shape
-        if e is not None:
-            assert e.dtype == torch.float32, "error_buf must be float32"
-            assert e.shape == (n, k), f"error_buf shape {tuple(e.shape)} != weight shape {(n, k)}"
-            assert e.is_contiguous(), "error_buf must be contiguous"
-        hi = torch.empty((n, k), dtype=torch.float8_e4m3fn, device=dev)
-        lo = torch.empty((n, k), dtype=torch.float8_e4m3fn, device=dev)
-        ih = torch.empty(1, dtype=torch.float32, device=dev)
-        il = torch.empty(1, dtype=torch.float32, device=dev)
-        ht = torch.empty((k, n), dtype=torch.float8_e4m3fn, device=dev) if t else None
-        lt = torch.empty((k, n), dtype=torch.float8_e4m3fn, device=dev) if t else None
-        jobs[i] = _hip.QuantJob(_hip.JOB_DUAL, ptr(w), _in_dtype(w), n, k, ptr(e), int(bool(u)),
-                                0, ptr(hi), ptr(ht), ptr(ih), ptr(lo), ptr(lt), ptr(il))
-        res_d.append((hi, lo, ih, il, ht, lt) if t else (hi, lo, ih, il))
-    for i, (x, f, t) in enumerate(act, start=len(dual)):
-        x = x if x.is_contiguous() else x.contiguous()
-        rows, cols = x.shape
-        q = torch.empty((rows, cols), dtype=f, device=dev)
-        qt = torch.empty((cols, rows), dtype=f, device=dev) if t else None
-        inv = torch.empty(1, dtype=torch.float32, device=dev)
-        jobs[i] = _hip.QuantJob(_hip.JOB_ACT, ptr(x), _in_dtype(x), rows, cols, None, 0, _fmt(f),
-                                ptr(q), ptr(qt), ptr(inv), None, None, None)
-        res_a.append((q, inv, qt) if t else (q, inv))
-    ws = _hip.batch_workspace(dev)
-    check(_hip.lib().tcfp_quantize_batch(len(jobs), jobs, ptr(ws), ws.numel(),
-                                         _hip.stream_of(dev)), "quantize_batch")
-    return res_d, res_a
+    return _hip.host().quantize_batch(dual, act)
 
 
 def _dual_quantize_nf(w, n, k, error_buf, update_ef, sigma_factor, stochastic_hi, stochastic_lo,
@@ -576,45 +491,7 @@ def _gemm_operand(t: torch.Tensor, name: str) -> torch.Tensor:
 
 
 def _dual_gemm(a, b_hi, b_lo, s_a, s_hi, s_lo, bias, out_dtype):
-    dev = _hip.require_gpu(a, b_hi, b_lo, s_a, s_hi, s_lo, bias)
-    a = _gemm_operand(a, "A")
-    b_hi = _gemm_operand(b_hi, "B_hi")
-    b_lo = _gemm_operand(b_lo, "B_lo") if b_lo is not None else None
-    m, k = a.shape
-    n = b_hi.shape[0]
-    if k % 16 != 0:
-        raise ValueError(f"K ({k}) must be divisible by 16")
-    if b_hi.stride(0) != (b_lo.stride(0) if b_lo is not None else b_hi.stride(0)):
-        b_lo = b_lo.contiguous()
-        b_hi = b_hi.contiguous()
-    out = torch.empty((m, n), dtype=out_dtype, device=dev)
-    if bias is not None:
-        bias = _bias_f32(bias, n)
-    check(
-        _hip.lib().tcfp_dual_gemm(
-            ptr(a), _fmt(a.dtype), a.stride(0), ptr(b_hi), ptr(b_lo), _fmt(b_hi.dtype),
-            b_hi.stride(0), m, n, k, ptr(_scalar(s_a, "scale_a")), ptr(_scalar(s_hi, "scale_hi")),
-            ptr(_scalar(s_lo, "scale_lo")) if s_lo is not None else None, ptr(bias), ptr(out),
-            _out_dtype(out_dtype), n, _hip.stream_of(dev),
-        ),
-        "dual_gemm",
-    )
-    return out
-
-
-def _gemm_operands(a, b_hi, b_lo):
-    a = _gemm_operand(a, "A")
-    b_hi = _gemm_operand(b_hi, "B_hi")
-    b_lo = _gemm_operand(b_lo, "B_lo")
-    if a.shape[1] != b_hi.shape[1] or b_hi.shape != b_lo.shape:
-        raise AssertionError(
-            f"Shape mismatch: A{tuple(a.shape)}, B_hi{tuple(b_hi.shape)}, B_lo{tuple(b_lo.shape)}"
-        )
-    if a.shape[1] % 16 != 0:
-        raise ValueError(f"K ({a.shape[1]}) must be divisible by 16")
-    if b_hi.stride(0) != b_lo.stride(0):
-        b_hi, b_lo = b_hi.contiguous(), b_lo.contiguous()
-    return a, b_hi, b_lo
+    return _hip.host().dual_gemm(a, b_hi, b_lo, s_a, s_hi, s_lo, bias, out_dtype)
 
 
 def dual_gemm_gelu_quantize(
@@ -642,39 +519,9 @@ def dual_gemm_gelu_quantize(
     when ``return_act``, then the GELU derivative factor when
     ``return_dgelu`` (what ``dual_gemm_dgelu_quantize_colsum`` takes).
     """
-    dev = _hip.require_gpu(act_fp8, w_hi_fp8, w_lo_fp8, act_inv, w_hi_inv, w_lo_inv, bias)
-    a, b_hi, b_lo = _gemm_operands(act_fp8, w_hi_fp8, w_lo_fp8)
-    m, k = a.shape
-    n = b_hi.shape[0]
-    if return_dgelu and n % 8 != 0:
-        raise ValueError(f"return_dgelu needs N divisible by 8, got {n}")
-    h = torch.empty((m, n), dtype=torch.float32, device=dev)
-    store = return_act or n % 8 != 0
-    act = torch.empty((m, n), dtype=torch.float32, device=dev) if store else None
-    dg = torch.empty((m, n), dtype=torch.float32, device=dev) if return_dgelu else None
-    q = torch.empty((m, n), dtype=fp8_dtype, device=dev)
-    q_t = torch.empty((n, m), dtype=fp8_dtype, device=dev) if transpose else None
-    inv = torch.empty(1, dtype=torch.float32, device=dev)
-    if bias is not None:
-        bias = _bias_f32(bias, n)
-    check(
-        _hip.lib().tcfp_dual_gemm_gelu_quantize(
-            ptr(a), _fmt(a.dtype), a.stride(0), ptr(b_hi), ptr(b_lo), _fmt(b_hi.dtype),
-            b_hi.stride(0), m, n, k, ptr(_scalar(act_inv, "scale_a")),
-            ptr(_scalar(w_hi_inv, "scale_hi")), ptr(_scalar(w_lo_inv, "scale_lo")), ptr(bias),
-            ptr(h), ptr(act), ptr(dg), _fmt(fp8_dtype), ptr(q), ptr(q_t), ptr(inv),
-            ptr(_hip.workspace(dev)), _hip.stream_of(dev),
-        ),
-        "dual_gemm_gelu_quantize",
-    )
-    out = (h, q, inv)
-    if transpose:
-        out = out + (q_t,)
-    if return_act:
-        out = out + (act,)
-    if return_dgelu:
-        out = out + (dg,)
-    return out
+    return _hip.host().dual_gemm_gelu_quantize(
+        act_fp8, w_hi_fp8, w_lo_fp8, act_inv, w_hi_inv, w_lo_inv, bias, fp8_dtype, transpose,
+        return_act, return_dgelu)
 
 
 def gelu_amax_rule_status() -> tuple[bool, bool, float]:
@@ -720,41 +567,9 @@ def dual_gemm_dgelu_quantize_colsum(
     """
     if not codes and not transpose:
         raise ValueError("codes=False needs transpose=True (the codes are written one way or both)")
-    dev = _hip.require_gpu(grad_fp8, w_hi_t, w_lo_t, grad_inv, w_hi_inv, w_lo_inv, dgelu)
-    a, b_hi, b_lo = _gemm_operands(grad_fp8, w_hi_t, w_lo_t)
-    m, k = a.shape
-    n = b_hi.shape[0]
-    if dgelu.dtype != torch.float32 or tuple(dgelu.shape) != (m, n):
-        raise AssertionError(
-            f"dgelu must be float32 of shape {(m, n)}, got {dgelu.dtype} {tuple(dgelu.shape)}")
-    if n % 8 != 0:
-        raise ValueError(f"column count ({n}) must be divisible by 8")
-    dc = dgelu if dgelu.is_contiguous() else dgelu.contiguous()
-    g = torch.empty((m, n), dtype=torch.float32, device=dev)
-    q = torch.empty((m, n), dtype=fp8_dtype, device=dev) if codes else None
-    q_t = torch.empty((n, m), dtype=fp8_dtype, device=dev) if transpose else None
-    inv = torch.empty(1, dtype=torch.float32, device=dev)
-    cs = torch.empty(n, dtype=torch.float32, device=dev) if col_sum else None
-    nbytes = int(_hip.lib().tcfp_colsum_workspace_bytes(m, n)) if col_sum else 0
-    cws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev) if col_sum else None
-    check(
-        _hip.lib().tcfp_dual_gemm_dgelu_quantize_colsum(
-            ptr(a), _fmt(a.dtype), a.stride(0), ptr(b_hi), ptr(b_lo), _fmt(b_hi.dtype),
-            b_hi.stride(0), m, n, k, ptr(_scalar(grad_inv, "scale_a")),
-            ptr(_scalar(w_hi_inv, "scale_hi")), ptr(_scalar(w_lo_inv, "scale_lo")), ptr(dc),
-            ptr(g), _fmt(fp8_dtype), ptr(q), ptr(q_t), ptr(inv), ptr(cs),
-            ptr(_hip.workspace(dev)), ptr(cws), nbytes, _hip.stream_of(dev),
-        ),
-        "dual_gemm_dgelu_quantize_colsum",
-    )
-    out = (q, inv)
-    if transpose:
-        out = out + (q_t,)
-    if col_sum:
-        out = out + (cs,)
-    if return_grad:
-        out = out + (g,)
-    return out
+    return _hip.host().dual_gemm_dgelu_quantize_colsum(
+        grad_fp8, w_hi_t, w_lo_t, grad_inv, w_hi_inv, w_lo_inv, dgelu, fp8_dtype, transpose,
+        col_sum, return_grad, codes)
 
 
 def fused_dual_gemm_forward(
@@ -868,22 +683,7 @@ def block_quantize_fp8(
     fp8 * multiplier.
     """
     f32s = _scale_format(scale_format)
-    dev = _hip.require_gpu(tensor)
-    M, K = tensor.shape
-    assert K % block_size == 0, f"K ({K}) must be divisible by block_size ({block_size})"
-    if block_size not in (32, 64, 128):
-        raise ValueError(f"block_size must be 32, 64, or 128, got {block_size}")
-    x = tensor if tensor.is_contiguous() else tensor.contiguous()
-    q = torch.empty((M, K), dtype=fp8_dtype, device=dev)
-    scales = torch.empty((K // block_size, M), dtype=torch.float32 if f32s else torch.int8,
-                         device=dev)
-    fn = _hip.lib().tcfp_block_quantize_f32s if f32s else _hip.lib().tcfp_block_quantize
-    check(
-        fn(ptr(x), _in_dtype(x), M, K, block_size, _fmt(fp8_dtype), ptr(q), ptr(scales),
-           _hip.stream_of(dev)),
-        "block_quantize_fp8",
-    )
-    return q, scales
+    return _hip.host().block_quantize(tensor, block_size, fp8_dtype, f32s)
 
 
 def block_dequantize_fp8(
@@ -985,37 +785,7 @@ def _block_exps(e: torch.Tensor, rows: int, num_kb: int, name: str,
 
 
 def _block_gemm(a, e_a, b_hi, b_lo, e_hi, e_lo, block_size, bias, out_dtype):
-    dev = _hip.require_gpu(a, e_a, b_hi, b_lo, e_hi, e_lo, bias)
-    a = _gemm_operand(a, "A")
-    b_hi = _gemm_operand(b_hi, "B_hi")
-    b_lo = _gemm_operand(b_lo, "B_lo") if b_lo is not None else None
-    m, k = a.shape
-    n = b_hi.shape[0]
-    assert k % block_size == 0, f"K ({k}) not divisible by block_size ({block_size})"
-    if block_size not in (32, 64, 128):
-        raise ValueError(f"block_size must be 32, 64, or 128, got {block_size}")
-    num_kb = k // block_size
-    # int8 exponents (the reference's format) or fp32 multipliers, not mixed
-    sdt = torch.float32 if e_a.dtype == torch.float32 else torch.int8
-    e_a = _block_exps(e_a, m, num_kb, "scales_a", sdt)
-    e_hi = _block_exps(e_hi, n, num_kb, "scales_b", sdt)
-    e_lo = _block_exps(e_lo, n, num_kb, "scales_lo", sdt) if b_lo is not None else None
-    if b_lo is not None and b_hi.stride(0) != b_lo.stride(0):
-        b_hi, b_lo = b_hi.contiguous(), b_lo.contiguous()
-    out = torch.empty((m, n), dtype=out_dtype, device=dev)
-    if bias is not None:
-        bias = _bias_f32(bias, n)
-    fn = (_hip.lib().tcfp_block_dual_gemm_f32s if sdt == torch.float32
-          else _hip.lib().tcfp_block_dual_gemm)
-    check(
-        fn(
-            ptr(a), _fmt(a.dtype), a.stride(0), ptr(e_a), ptr(b_hi), ptr(b_lo),
-            _fmt(b_hi.dtype), b_hi.stride(0), ptr(e_hi), ptr(e_lo), m, n, k, block_size,
-            ptr(bias), ptr(out), _out_dtype(out_dtype), n, _hip.stream_of(dev),
-        ),
-        "block_dual_gemm",
-    )
-    return out
+    return _hip.host().block_gemm(a, e_a, b_hi, b_lo, e_hi, e_lo, block_size, bias, out_dtype)
 
 
 def block_scaled_gemm(
@@ -1085,49 +855,9 @@ def block_linear_forward(x2d, weight, bias, block_size, error_buf=None, srr=Fals
     small host-bound models see).  ``x2d`` [M, K] fp32/bf16, ``weight``
     [N, K] contiguous.  Returns ``(out fp32 [M, N], w_hi, w_lo, e_hi, e_lo,
     act_fp8, act_e)``."""
-    bs = block_size
-    if bs not in (32, 64, 128):
-        raise ValueError(f"block_size must be 32, 64, or 128, got {bs}")
-    M, Kd = x2d.shape
-    N = weight.shape[0]
-    assert weight.is_contiguous() and weight.shape[1] == Kd and Kd % bs == 0, (
-        f"weight {tuple(weight.shape)} vs input ({M}, {Kd}), block {bs}")
-    if srr and error_buf is not None:
-        raise ValueError("stochastic_lo and error_buf are mutually exclusive")
-    dev = _hip.require_gpu(x2d, weight, error_buf, bias)
-    lib = _hip.lib()
-    st = _hip.stream_of(dev)
-    nkb = Kd // bs
-    e4 = torch.float8_e4m3fn
-    w_hi = torch.empty((N, Kd), dtype=e4, device=dev)
-    w_lo = torch.empty((N, Kd), dtype=e4, device=dev)
-    e_hi = torch.empty((nkb, N), dtype=torch.int8, device=dev)
-    e_lo = torch.empty((nkb, N), dtype=torch.int8, device=dev)
     seed = int(torch.randint(0, 2**62, (1,)).item()) if srr else 0
-    check(lib.tcfp_block_dual_quantize(
-        ptr(weight), _in_dtype(weight), N, Kd, bs, ptr(error_buf), int(bool(update_ef)),
-        int(bool(srr)), seed, 0, ptr(w_hi), ptr(w_lo), ptr(e_hi), ptr(e_lo), st),
-        "fused_dual_quantize_fp8")
-    act = x2d
-    if not act.is_contiguous() or act.data_ptr() % 16 != 0:
-        act = act.contiguous()
-    b = _bias_f32(bias, N) if bias is not None else None
-    out = torch.empty((M, N), dtype=torch.float32, device=dev)
-    act_fp8 = torch.empty((M, Kd), dtype=e4, device=dev)
-    act_e = torch.empty((nkb, M), dtype=torch.int8, device=dev)
-    if (N + 127) // 128 <= 4:
-        check(lib.tcfp_act_quant_block_dual_gemm(
-            ptr(act), _in_dtype(act), Kd, ptr(w_hi), ptr(w_lo), Kd, ptr(e_hi), ptr(e_lo), M, N,
-            Kd, bs, ptr(b), ptr(out), N, ptr(act_fp8), ptr(act_e), st),
-            "fused_act_quant_dual_gemm_forward")
-    else:
-        check(lib.tcfp_block_quantize(ptr(act), _in_dtype(act), M, Kd, bs, FP8_E4M3,
-                                      ptr(act_fp8), ptr(act_e), st), "block_quantize_fp8")
-        check(lib.tcfp_block_dual_gemm(
-            ptr(act_fp8), FP8_E4M3, Kd, ptr(act_e), ptr(w_hi), ptr(w_lo), FP8_E4M3, Kd,
-            ptr(e_hi), ptr(e_lo), M, N, Kd, bs, ptr(b), ptr(out), DTYPE_F32, N, st),
-            "block_dual_gemm")
-    return out, w_hi, w_lo, e_hi, e_lo, act_fp8, act_e
+    return _hip.host().block_linear_forward(x2d, weight, bias, block_size, error_buf, srr,
+                                            update_ef, seed)
 
 
 def fused_block_scaled_dual_gemm_forward(
@@ -1480,9 +1210,6 @@ def block_backward_prep(
     return g_deq, g_split, bias_grad
 
 
-_BWD_WS: dict[tuple, tuple[int, int, int]] = {}
-
-
 def block_linear_backward(grad_2d, act_fp8, act_e, w_hi, w_lo, e_hi, e_lo, block_size,
                           need_dx, need_dw, want_db, split_lo=True):
     """The launches of a block-scaled TCFP layer's default backward, as
@@ -1498,49 +1225,8 @@ def block_linear_backward(grad_2d, act_fp8, act_e, w_hi, w_lo, e_hi, e_lo, block
     ``split_lo``); ``w_hi`` .. ``e_lo`` the forward's weight operands
     (``need_dx``).  Returns ``(dx fp32 [M, D_in], dw fp32 [D_out, D_in],
     db fp32 [D_out])``, None where not requested."""
-    bs = block_size
-    M, Nout = grad_2d.shape
-    Kin = w_hi.shape[1] if need_dx else (act_fp8.shape[1] if need_dw else 0)
-    dev = _hip.require_gpu(grad_2d, act_fp8, w_hi)
-    lib = _hip.lib()
-    st = _hip.stream_of(dev)
-    key = (M, Nout, Kin, bool(split_lo), bool(want_db), bool(need_dw), bool(need_dx))
-    sizes = _BWD_WS.get(key)
-    if sizes is None:
-        sizes = (int(lib.tcfp_block_grad_prep_workspace_bytes(M, Nout)) if want_db else 0,
-                 int(lib.tcfp_block_wgrad_presplit_workspace_bytes(M, Nout, Kin, int(split_lo)))
-                 if need_dw else 0,
-                 int(lib.tcfp_block_dual_gemm_dx_bf16_workspace_bytes(Nout, Kin)) if need_dx else 0)
-        _BWD_WS[key] = sizes
-    n_prep, n_w, n_d = sizes
-    g = grad_2d if (grad_2d.dtype == torch.float32 and grad_2d.is_contiguous()) else (
-        grad_2d.float().contiguous())
-    bf = torch.bfloat16
-    g_deq = torch.empty((M, Nout), dtype=bf, device=dev) if need_dx else None
-    g_split = (torch.empty((Nout, 2 * M if split_lo else M), dtype=bf, device=dev)
-               if need_dw else None)
-    db = torch.empty((Nout,), dtype=torch.float32, device=dev) if want_db else None
-    ws = torch.empty(max(n_prep, 1), dtype=torch.uint8, device=dev) if want_db else None
-    check(lib.tcfp_block_grad_prep(ptr(g), M, Nout, bs, ptr(g_deq), ptr(g_split), int(split_lo),
-                                   ptr(db), None, None, ptr(ws), n_prep, st),
-          "block_backward_prep")
-    # (the gradient copy and each scratch are released before the next
-    # allocation, as the per-op calls release theirs on return)
-    g = dw = dx = ws = None
-    if need_dw:
-        dw = torch.empty((Nout, Kin), dtype=torch.float32, device=dev)
-        ws = torch.empty(max(n_w, 1), dtype=torch.uint8, device=dev)
-        check(lib.tcfp_block_wgrad_presplit(
-            ptr(g_split), int(split_lo), M, Nout, ptr(act_fp8), _fmt(act_fp8.dtype), ptr(act_e),
-            Kin, bs, ptr(dw), ptr(ws), n_w, st), "block_wgrad_from_prep")
-    g_split = ws = None  # (released before dX is allocated)
-    if need_dx:
-        dx = torch.empty((M, Kin), dtype=torch.float32, device=dev)
-        ws = torch.empty(max(n_d, 1), dtype=torch.uint8, device=dev)
-        check(lib.tcfp_block_dual_gemm_dx_bf16(
-            ptr(g_deq), ptr(w_hi), ptr(w_lo), ptr(e_hi), ptr(e_lo), M, Nout, Kin, bs, ptr(dx),
-            ptr(ws), n_d, st), "block_dgrad_from_prep")
-    return dx, dw, db
+    return _hip.host().block_linear_backward(grad_2d, act_fp8, act_e, w_hi, w_lo, e_hi, e_lo,
+                                             block_size, need_dx, need_dw, want_db, split_lo)
 
 
 def block_dgrad_from_prep(g_deq, w_hi_fp8, w_lo_fp8, w_hi_scales, w_lo_scales, block_size):
