@@ -845,6 +845,59 @@ TCFP_DEV void gather_transpose(const uint32_t* tile, int rc, int c4, uint4 out[4
 #pragma unroll
     for (int qd = 0; qd < 4; ++qd) {
       const int sh = 8 * b;
+// Both passes of a small tensor in one workgroup: the values stay in registers
+// between the maximum and the codes, and the second launch and its gap
+// (which cost more than the work up to here) go.  Bound: one CU's reads.
+constexpr int kOneThreads = 1024;
+constexpr int kOneVecs = 4;  // 8-element vectors per thread
+constexpr int64_t kOneMax = int64_t(kOneThreads) * kOneVecs * 8;
+
+template <typename InT, int FMT>
+__global__ __launch_bounds__(kOneThreads) void quant_one_kernel(const InT* __restrict__ x,
+                                                                int64_t n, int bf16_rule,
+                                                                uint8_t* __restrict__ q,
+                                                                float* scale_out,
+                                                                float* inv_out) {
+  __shared__ uint32_t red[kOneThreads / 64];
+  const float mx = FMT == TCFP_FP8_E5M2 ? kE5M2Max : kE4M3Max;
+  const int nvec = int(n >> 3), tid = int(threadIdx.x);
+  const int t = nvec * 8 + tid;  // the last n % 8 elements
+  float v[kOneVecs][8], tail = 0.0f;
+  uint32_t m = 0;
+#pragma unroll
+  for (int u = 0; u < kOneVecs; ++u) {
+    const int i = u * kOneThreads + tid;
+    if (i < nvec) {
+      load8(x + int64_t(i) * 8, v[u]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[u][j] = 0.0f;
+    }
+  }
+  if (t < n) tail = load1(x + t);
+#pragma unroll
+  for (int u = 0; u < kOneVecs; ++u)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m = umax(m, absbits(v[u][j]));
+  m = block_umax_nt<kOneThreads>(umax(m, absbits(tail)), red);
+  float s, inv;
+  scale_from_amax(__uint_as_float(m), bf16_rule != 0, mx, &s, &inv);
+  if (tid == 0) {
+    if (scale_out) *scale_out = s;
+    if (inv_out) *inv_out = inv;
+  }
+#pragma unroll
+  for (int u = 0; u < kOneVecs; ++u) {
+    const int i = u * kOneThreads + tid;
+    if (i < nvec) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[u][j] = clampf(v[u][j] * s, mx);
+      *reinterpret_cast<uint2*>(q + int64_t(i) * 8) = encode8<FMT>(v[u]);
+    }
+  }
+  if (t < n) q[t] = uint8_t(encode1<FMT>(clampf(tail * s, mx)));
+}
+
       o[qd] = ((w[4 * qd] >> sh) & 0xFFu) | (((w[4 * qd + 1] >> sh) & 0xFFu) << 8) |
               (((w[4 * qd + 2] >> sh) & 0xFFu) << 16) | (((w[4 * qd + 3] >> sh) & 0xFFu) << 24);
     }
@@ -2300,6 +2353,20 @@ int quantize_impl(const void* x, int x_dtype, int64_t rows, int64_t cols, int fp
 }
 
 }  // namespace
+  // a small tensor without a transposed copy: one workgroup, one launch
+  if (!scale_in && pre_g == 0 && !gelu_in && !q_t && !col_sum && n <= kOneMax) {
+    if (!q && n > 0) return TCFP_ERR_SHAPE;
+#define TCFP_Q1(T, F)                                                                     \
+  quant_one_kernel<T, F><<<1, kOneThreads, 0, st>>>(static_cast<const T*>(x), n, bf ? 1 : 0, \
+                                                    q, scale_out, inv_out)
+    if (bf) {
+      if (fp8_fmt == TCFP_FP8_E5M2) TCFP_Q1(uint16_t, TCFP_FP8_E5M2); else TCFP_Q1(uint16_t, TCFP_FP8_E4M3);
+    } else {
+      if (fp8_fmt == TCFP_FP8_E5M2) TCFP_Q1(float, TCFP_FP8_E5M2); else TCFP_Q1(float, TCFP_FP8_E4M3);
+    }
+#undef TCFP_Q1
+    return launch_status();
+  }
 
 namespace tcfp {
 
