@@ -1,4 +1,5 @@
-"""Quantisation paths taken by size: the one-launch cast of small tensors."""
+"""Quantisation paths taken by size and by the data: the one-launch cast of
+small tensors and the candidate windows of flat weight distributions."""
 import numpy as np
 import pytest
 import torch
@@ -52,3 +53,43 @@ def test_small_cast_special_values(dev, bad):
     assert torch.equal(q.view(torch.uint8), qb.view(torch.uint8)[:1000])
     assert torch.equal(inv.isnan(), invb.isnan())
     assert torch.equal(inv.nan_to_num(), invb.nan_to_num())
+
+
+def _flat_case(name, shape, g):
+    w = torch.rand(shape, generator=g) * 2 - 1
+    if name == "rows":          # every row its own range: most maxima far below the amax
+        w = w * (0.6 + 0.4 * torch.rand(shape[0], 1, generator=g))
+    elif name == "late":        # the amax comes last, 2% above all before it
+        w = w * 0.98
+        w[-1, -1] = 1.0
+    elif name == "one_short":   # a tenth of a percent above: the windows still decide
+        w = w * 0.999
+        w[0, 0] = -1.0
+    elif name == "edges":       # values on the codes and the midpoints only
+        w = (256 + 16 * torch.randint(0, 13, shape, generator=g)).float() / 448
+    return w
+
+
+@pytest.mark.parametrize("name", ["uniform", "rows", "late", "one_short", "edges"])
+@pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("ef", [True, False])
+def test_candidate_windows_match_full_pass(dev, name, wdtype, ef):
+    """Flat distributions (the layers' initialisation) keep only the values near
+    a midpoint between codes; the results are the full pass's bit for bit,
+    where the windows decide and where the maxima lie too far apart."""
+    shape = (4096, 2056)
+    g = torch.Generator().manual_seed(len(name))
+    w = (_flat_case(name, shape, g) * 0.03).to(wdtype).to(dev)
+    e = (torch.randn(shape, generator=g) * 1e-6).to(dev) if ef else None
+    outs = []
+    try:
+        for on in (True, False):
+            K.set_dual_quant_candidates(on)
+            buf = e.clone() if ef else None
+            res = K.dual_quantize_per_tensor(w, buf, transposed=True)
+            outs.append([r.view(torch.uint8) if r.dtype.itemsize == 1 else r for r in res]
+                        + ([buf] if ef else []))
+    finally:
+        K.set_dual_quant_candidates(True)
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
