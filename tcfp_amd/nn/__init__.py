@@ -29,6 +29,7 @@ from __future__ import annotations
 import warnings
 
 import torch
+import torch.autograd.forward_ad as fwAD
 import torch.nn as nn
 import torch.nn.functional as F
 
@@ -50,6 +51,17 @@ __all__ = [
 
 def _flatten(t: torch.Tensor) -> torch.Tensor:
     return t.reshape(-1, t.shape[-1]) if t.ndim != 2 else t
+
+
+def _for_inference(*tensors):
+    """``tensors`` as a forward pass that records no graph takes them: detached
+    when autograd is off, since a Function's ``needs_input_grad`` follows
+    ``requires_grad`` alone, and the copies only a backward reads (transposed
+    codes, GELU factors) would be made for nothing.  Forward-mode AD also runs
+    with autograd off; inside its levels the tensors stay as they are."""
+    if torch.is_grad_enabled() or fwAD._current_level >= 0:
+        return tensors
+    return tuple(t.detach() if t is not None and t.requires_grad else t for t in tensors)
 
 
 def _ef_buffer(state: ErrorFeedbackState | None, name: str, weight: torch.Tensor):
@@ -498,13 +510,14 @@ class TCFPLinear(nn.Module):
             self._warmup_remaining -= 1
             return F.linear(x, self.weight, self.bias)
         update_ef = self._ef_update_flag()
+        x, weight, bias = _for_inference(x, self.weight, self.bias)
         if self.scale_block_size is not None:
             return _TCFP12BlockScaledFunction.apply(
-                x, self.weight, self.bias, self.scale_block_size, self.hp_grad_weight,
+                x, weight, bias, self.scale_block_size, self.hp_grad_weight,
                 self._error_state, self._param_name, self.abd, self.srr, update_ef,
             )
         return _TCFP12TensorCoreFunction.apply(
-            x, self.weight, self.bias, self.nf_aware_scaling, self.sigma_factor,
+            x, weight, bias, self.nf_aware_scaling, self.sigma_factor,
             self.stochastic_rounding, self.hp_grad_weight, self._error_state,
             self._param_name, self.delayed_scaling, self.use_fused_kernel, self.use_cuda_ext,
             self.abd, self.srr, update_ef,
@@ -717,7 +730,7 @@ class TCFPMLP(nn.Sequential):
         u1 = fc1._ef_update_flag()
         u2 = fc2._ef_update_flag()
         return _TCFP12FusedMLPFunction.apply(
-            x, fc1.weight, fc1.bias, fc2.weight, fc2.bias,
+            *_for_inference(x, fc1.weight, fc1.bias, fc2.weight, fc2.bias),
             fc1._error_state, fc1._param_name, fc2._error_state, fc2._param_name, u1, u2,
         )
 

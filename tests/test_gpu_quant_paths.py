@@ -1,12 +1,15 @@
 """Quantisation paths taken by size and by the data: the one-launch cast of
-small tensors and the candidate windows of flat weight distributions."""
+small tensors, the candidate windows of flat weight distributions, and the
+layers' forward without autograd."""
 import numpy as np
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 
 from oracle import fp8 as ofp8
 from oracle import quant as oq
 from tcfp_amd import kernels as K
+from tcfp_amd.nn import TCFPLinear, fuse_tcfp_mlp
 
 pytestmark = pytest.mark.gpu
 
@@ -93,3 +96,38 @@ def test_candidate_windows_match_full_pass(dev, name, wdtype, ef):
         K.set_dual_quant_candidates(True)
     for x, y in zip(*outs):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("kw,d", [({}, 256), ({"scale_block_size": 64}, 1024), ({}, 2944)])
+def test_forward_without_autograd_makes_no_backward_copies(dev, kw, d):
+    """Under no_grad: the values of the recording forward, no transposed codes
+    (d = 2944: the weight beyond the batch's size), parameters untouched, and
+    forward-mode AD still refused."""
+    torch.manual_seed(0)
+    layer = TCFPLinear(d, d, use_tensor_cores=True, **kw).to(dev)
+    x = torch.randn(48, d, device=dev, requires_grad=True)
+    ref = layer(x)
+    layer._last_weight_version = -1  # the EF buffer the recording forward wrote
+    layer._error_state.reset()
+    with torch.no_grad():
+        out = layer(x)
+        names = _kernel_names(lambda: layer(x))
+    assert torch.equal(out, ref.detach()) and not out.requires_grad
+    assert not any("dualq_lo_t" in k for k in names)
+    assert layer.weight.requires_grad and x.requires_grad
+    with torch.no_grad(), fwAD.dual_level(), pytest.raises(RuntimeError):
+        layer(fwAD.make_dual(x.detach(), torch.ones_like(x)))
+
+
+def test_mlp_without_autograd(dev):
+    torch.manual_seed(0)
+    mlp = fuse_tcfp_mlp(torch.nn.Sequential(
+        TCFPLinear(256, 512, use_tensor_cores=True), torch.nn.GELU(),
+        TCFPLinear(512, 256, use_tensor_cores=True))).to(dev)
+    x = torch.randn(64, 256, device=dev)
+    ref = mlp(x)
+    for m in (mlp[0], mlp[2]):
+        m._error_state.reset()
+    with torch.no_grad():
+        out = mlp(x)
+    assert torch.equal(out, ref.detach()) and not out.requires_grad
