@@ -572,6 +572,18 @@ int tcfp_block_wgrad(const float* g, int64_t m, int64_t n_out, const uint8_t* x,
                      const int8_t* e_x, int64_t k_in, int block, float* dw, void* workspace,
                      size_t workspace_bytes, void* stream);
 
+/* dW = g^T deq(x) to fp32 accuracy for any token count m >= 1: g [m, n_out]
+ * fp32 (16-byte aligned), x [m, k_in] FP8 codes (k_in % 16 == 0) with a
+ * per-tensor inverse scale `inv` (device scalar; NULL: 1) or block exponents
+ * e_x [k_in / block, m] (NULL: none).  The fp32 matmuls that the reference
+ * runs where its FP8 product does not apply (tcfp/nn/__init__.py:553-555,
+ * 743-750), as three exact bf16 passes.  dw [n_out, k_in] fp32.  Workspace:
+ * tcfp_wgrad_f32_workspace_bytes(m, n_out, k_in). */
+size_t tcfp_wgrad_f32_workspace_bytes(int64_t m, int64_t n_out, int64_t k_in);
+int tcfp_wgrad_f32(const float* g, int64_t m, int64_t n_out, const uint8_t* x, int x_fmt,
+                   const float* inv, const int8_t* e_x, int64_t k_in, int block, float* dw,
+                   void* workspace, size_t workspace_bytes, void* stream);
+
 /* Block backward, fused operand preparation (no single reference
  * counterpart: it produces, in one pass over the fp32 gradient g [m, n],
  * what the reference's backward derives from it separately,

@@ -132,6 +132,9 @@ _SIGNATURES = {
                                      _i64, _i64, _i32, _c_void_p, _c_void_p, ctypes.c_size_t,
                                      _c_void_p],
     "tcfp_block_dual_gemm_dx_bf16_workspace_bytes": [_i64, _i64],
+    "tcfp_wgrad_f32_workspace_bytes": [_i64, _i64, _i64],
+    "tcfp_wgrad_f32": [_c_void_p, _i64, _i64, _c_void_p, _i32, _c_void_p, _c_void_p, _i64, _i32,
+                       _c_void_p, _c_void_p, ctypes.c_size_t, _c_void_p],
     "tcfp_block_wgrad_presplit": [_c_void_p, _i32, _i64, _i64, _c_void_p, _i32, _c_void_p, _i64,
                                   _i32, _c_void_p, _c_void_p, ctypes.c_size_t, _c_void_p],
     "tcfp_block_wgrad_presplit_workspace_bytes": [_i64, _i64, _i64, _i32],
@@ -153,6 +156,7 @@ _RESTYPE = {
     "tcfp_block_grad_prep_workspace_bytes": ctypes.c_size_t,
     "tcfp_block_dual_gemm_dx_bf16_workspace_bytes": ctypes.c_size_t,
     "tcfp_block_wgrad_presplit_workspace_bytes": ctypes.c_size_t,
+    "tcfp_wgrad_f32_workspace_bytes": ctypes.c_size_t,
     "tcfp_quantize_batch_workspace_bytes": ctypes.c_size_t,
 }
 

@@ -246,9 +246,9 @@ struct GemmArgs {
   int kc;
   int64_t split_stride;
   // (gemm_nt_dma_kernel) kwrap_b > 0: the B operand rows hold kwrap_b bytes
-  // of contraction and byte k >= kwrap_b reads byte k - kwrap_b (K <= 2
-  // kwrap_b, kwrap_b % 128 == 0): one copy serves a contraction that runs
-  // over the same B columns twice
+  // of contraction and byte k reads byte k modulo kwrap_b (K <= 3 kwrap_b,
+  // kwrap_b % 128 == 0): one copy serves a contraction that runs over the
+  // same B columns two or three times
   int kwrap_b;
   // GELU epilogues of the persistent fp32 kernel (same leading dimension
   // ldo as out; EPI 2 ignores bias).  EPI 1 writes out (= h) as EPI 0 and the GELU amax rule's
@@ -523,6 +523,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
     uint32_t soff = uint32_t(live ? t : 0) * kSK;
     if (kwrap) {
       soff += uint32_t(koff);
+      if (soff >= kwrap) soff -= kwrap;
       if (soff >= kwrap) soff -= kwrap;
     }
     const bool last = t == nt - 1;
@@ -1094,6 +1095,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
       if (kwrap) {
         soff += uint32_t(koff);
         if (soff >= kwrap) soff -= kwrap;
+        if (soff >= kwrap) soff -= kwrap;
       }
       uint32_t dst = lds_base + uint32_t(buf(tr)) * STAGE;
       uint32_t vo[DI];
@@ -1190,7 +1192,7 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   float c0s = 1.0f, c1s = 1.0f;
   if (SCALE == 0 && g.s_a) {
     const float sa = *g.s_a;
-    c0s = sa * *g.s_0;
+    c0s = g.s_0 ? sa * *g.s_0 : sa;
     c1s = SPLIT ? c0s : sa * *g.s_1;
   }
   const bool vec = (g.ldo % (16 / EB)) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
@@ -3272,8 +3274,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // contraction so every CU gets a workgroup, keeping at least four 128-byte
 // stages per split.  Returns the split count and sets *kc to the split
 // length in bytes (a multiple of 128).
-int64_t wgrad_splits(int64_t m, int64_t n_out, int64_t k_in, int64_t* kc, bool lo = true) {
-  const int64_t kbytes = (lo ? 4 : 2) * m;
+int64_t wgrad_splits_of(int64_t kbytes, int64_t n_out, int64_t k_in, int64_t* kc) {
   *kc = kbytes;
   const int64_t tiles = ((n_out + 127) / 128) * ((k_in + 127) / 128);
   const int64_t cus = num_cus();
@@ -3282,6 +3283,10 @@ int64_t wgrad_splits(int64_t m, int64_t n_out, int64_t k_in, int64_t* kc, bool l
   if (s < 2) return 1;
   *kc = ((kbytes + s - 1) / s + 127) / 128 * 128;
   return (kbytes + *kc - 1) / *kc;
+}
+
+int64_t wgrad_splits(int64_t m, int64_t n_out, int64_t k_in, int64_t* kc, bool lo = true) {
+  return wgrad_splits_of((lo ? 4 : 2) * m, n_out, k_in, kc);
 }
 
 // The wgrad GEMM over the concatenated contraction: A' = [g_hi | g_lo]^T
@@ -3383,6 +3388,143 @@ int wgrad_chunked(const uint16_t* ap, int64_t m, int64_t n_out, const uint8_t* x
     if (rc != TCFP_OK) return rc;
   }
   return TCFP_OK;
+}
+
+// ---- fp32-exact wgrad for any token count -----------------------------------
+// dW = G^T deq(X) with G in fp32 and X in FP8 codes, for the token counts that
+// the FP8 wgrad (m % 16) or the split-bf16 one (m % 4) do not take.  An fp32
+// significand is three bf16 ones: g = g1 + g2 + g3 by truncation, exactly, and
+// an FP8 code (times its block's power of two) is exact in bf16, so the
+// product is three bf16 passes over one copy of X with fp32 accumulation,
+//   A' = [g1 | g2 | g3]^T  [n_out, 3 mp],   B' = x^T  [k_in, mp],
+// mp = m rounded up to 64 (zeros behind), where an fp32 matrix product runs
+// at a sixteenth of the bf16 rate.  A per-tensor scale goes into the epilogue.
+// (With the dequantising copies of the fp32 form: 1000 tokens, 1040 -> 1552,
+// 53 -> 40 us; 2000 tokens, 4096 -> 8192, 936 -> 473; 1999 tokens, 1024 -> 4096,
+// 138 -> 75; 201 tokens, 256 -> 512, 31 -> 18.5.  Errors against 64 bits 1e-7
+// where the fp32 product's are 6e-7.)
+
+// out[c, j mp + r] = part j + 1 of g[r, c] (r < mp; rows past m zero); the
+// grid's columns start at c_base, out's rows at 0.
+__global__ __launch_bounds__(256) void split3_t_bf16_kernel(const float* __restrict__ g, int64_t m,
+                                                            int64_t n, int64_t c_base,
+                                                            int64_t c_count, int64_t mp,
+                                                            uint16_t* __restrict__ out) {
+  __shared__ float tile[64][64 + 1];
+  const int tiles_c = int((c_count + 63) / 64);
+  const int64_t r0 = int64_t(blockIdx.x / tiles_c) * 64, c0 = int64_t(blockIdx.x % tiles_c) * 64;
+  const int t = threadIdx.x;
+  // 16 lanes cover a row's 64 columns, 16 rows a pass
+  const int lc4 = (t & 15) * 4;
+#pragma unroll
+  for (int it = 0; it < 4; ++it) {
+    const int lr = it * 16 + (t >> 4);
+    const int64_t r = r0 + lr, c = c0 + lc4;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (r < m) {
+      const float* p = g + r * n + c_base + c;
+      if (n % 4 == 0 && c_base % 4 == 0 && c + 3 < c_count) {
+        const float4 a = *reinterpret_cast<const float4*>(p);
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (c + j < c_count) v[j] = p[j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tile[lc4 + j][lr] = v[j];
+  }
+  __syncthreads();
+  const int lc = t >> 2, lr = (t & 3) * 16;
+  const int64_t c = c0 + lc;
+  if (c >= c_count) return;
+  uint32_t w[3][8];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const float x = tile[lc][lr + j];
+    const uint32_t b = __float_as_uint(x);
+    uint32_t p1 = b >> 16, p2 = 0, p3 = 0;
+    if ((b & 0x7F800000u) != 0x7F800000u) {
+      const float x2 = x - __uint_as_float(b & 0xFFFF0000u);  // exact
+      const uint32_t b2 = __float_as_uint(x2);
+      p2 = b2 >> 16;
+      p3 = __float_as_uint(x2 - __uint_as_float(b2 & 0xFFFF0000u)) >> 16;  // exact, 8 bits
+    } else if ((b & 0x7FFFFFu) != 0) {
+      p1 = 0x7FC0u;  // a NaN stays one
+    }
+    const uint32_t p[3] = {p1, p2, p3};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      if (j & 1) w[q][j >> 1] |= p[q] << 16;
+      else w[q][j >> 1] = p[q];
+    }
+  }
+  uint16_t* o = out + c * (3 * mp) + r0 + lr;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    uint4* d = reinterpret_cast<uint4*>(o + q * mp);
+    d[0] = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
+    d[1] = make_uint4(w[q][4], w[q][5], w[q][6], w[q][7]);
+  }
+}
+
+// out[c, r] = bf16(q[r, c] * 2^e[c / bs, r]) (e null: the codes' values), r <
+// mp, rows past m zero.
+template <int FMT>
+__global__ __launch_bounds__(256) void codes_t_bf16_kernel(const uint8_t* __restrict__ q,
+                                                           const int8_t* __restrict__ e,
+                                                           int64_t m, int64_t k, int bs_shift,
+                                                           int64_t mp, bool vec,
+                                                           uint16_t* __restrict__ out) {
+  __shared__ uint16_t tile[64][64 + 2];
+  const int tiles_c = int((k + 63) / 64);
+  const int64_t r0 = int64_t(blockIdx.x / tiles_c) * 64, c0 = int64_t(blockIdx.x % tiles_c) * 64;
+  const int t = threadIdx.x;
+  {
+    const int lr = t >> 2, lc = (t & 3) * 16;
+    const int64_t r = r0 + lr;
+    if (vec && r < m && c0 + lc + 16 <= k) {
+      const uint4 w = *reinterpret_cast<const uint4*>(q + r * k + c0 + lc);
+      deq16_to_tile<FMT>(w, e ? exp2i(e[((c0 + lc) >> bs_shift) * m + r]) : 1.0f, tile, lc, lr);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int64_t c = c0 + lc + j;
+        uint16_t v = 0;
+        if (r < m && c < k)
+          v = f32_to_bf16_rne(fp8_to_f32<FMT>(q[r * k + c]) *
+                              (e ? exp2i(e[(c >> bs_shift) * m + r]) : 1.0f));
+        tile[lc + j][lr] = v;
+      }
+    }
+  }
+  __syncthreads();
+  const int lc = t >> 2, lr = (t & 3) * 16;
+  const int64_t c = c0 + lc;
+  if (c >= k) return;
+  uint32_t w[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    w[j] = uint32_t(tile[lc][lr + 2 * j]) | (uint32_t(tile[lc][lr + 2 * j + 1]) << 16);
+  uint4* o = reinterpret_cast<uint4*>(out + c * mp + r0 + lr);
+  o[0] = make_uint4(w[0], w[1], w[2], w[3]);
+  o[1] = make_uint4(w[4], w[5], w[6], w[7]);
+}
+
+int64_t f32w_mp(int64_t m) { return (m + 63) / 64 * 64; }
+// rows of dW per chunk: their split gradient stays within kOperandChunkBytes
+int64_t f32w_rows(int64_t m, int64_t n_out) { return chunk_cols(6 * f32w_mp(m), n_out); }
+size_t f32w_part_bytes(int64_t m, int64_t rows, int64_t k_in) {
+  int64_t kc;
+  const int64_t s = wgrad_splits_of(6 * f32w_mp(m), rows, k_in, &kc);
+  return s > 1 ? align256(size_t(s) * size_t(rows) * size_t(k_in) * 4) : 0;
+}
+size_t f32w_ws_bytes(int64_t m, int64_t n_out, int64_t k_in) {
+  const int64_t mp = f32w_mp(m), rows = f32w_rows(m, n_out);
+  const int64_t rem = rows > 0 ? n_out % rows : 0;
+  return align256(size_t(k_in) * size_t(mp) * 2) + align256(size_t(rows) * size_t(mp) * 6) +
+         std::max(f32w_part_bytes(m, rows, k_in), rem ? f32w_part_bytes(m, rem, k_in) : 0);
 }
 
 // ---- fused gradient preparation for the block backward ---------------------
@@ -3670,4 +3812,69 @@ extern "C" int tcfp_block_wgrad_presplit(const uint16_t* g_split_t, int split_lo
   const int shift = block == 32 ? 5 : (block == 64 ? 6 : 7);
   return wgrad_chunked(g_split_t, m, n_out, x, x_fmt, e_x, k_in, shift, dw,
                        static_cast<uint8_t*>(workspace), st, split_lo != 0);
+}
+
+extern "C" size_t tcfp_wgrad_f32_workspace_bytes(int64_t m, int64_t n_out, int64_t k_in) {
+  if (m < 0 || n_out < 0 || k_in < 0) return 0;
+  return f32w_ws_bytes(m, n_out, k_in);
+}
+
+extern "C" int tcfp_wgrad_f32(const float* g, int64_t m, int64_t n_out, const uint8_t* x, int x_fmt,
+                              const float* inv, const int8_t* e_x, int64_t k_in, int block,
+                              float* dw, void* workspace, size_t workspace_bytes, void* stream) {
+  if (m <= 0 || n_out < 0 || k_in < 0 || n_out > INT32_MAX || k_in > INT32_MAX ||
+      6 * f32w_mp(m) > INT32_MAX)
+    return TCFP_ERR_SHAPE;
+  if (k_in % 16 != 0) return TCFP_ERR_SHAPE;
+  if (e_x && ((block != 32 && block != 64 && block != 128) || k_in % block != 0))
+    return TCFP_ERR_SHAPE;
+  if (x_fmt != TCFP_FP8_E4M3 && x_fmt != TCFP_FP8_E5M2) return TCFP_ERR_DTYPE;
+  if (!g || !x || !dw) return TCFP_ERR_SHAPE;
+  if (n_out == 0 || k_in == 0) return TCFP_OK;
+  if (!workspace || workspace_bytes < f32w_ws_bytes(m, n_out, k_in)) return TCFP_ERR_WORKSPACE;
+  if (!al16(workspace) || !al16(dw) || !al16(g)) return TCFP_ERR_ALIGN;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t mp = f32w_mp(m), rows = f32w_rows(m, n_out);
+  const int shift = block == 32 ? 5 : (block == 64 ? 6 : 7);
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  uint16_t* xt = reinterpret_cast<uint16_t*>(ws);
+  ws += align256(size_t(k_in) * size_t(mp) * 2);
+  uint16_t* gs = reinterpret_cast<uint16_t*>(ws);
+  float* part = reinterpret_cast<float*>(ws + align256(size_t(rows) * size_t(mp) * 6));
+  const int64_t tx = (mp / 64) * ((k_in + 63) / 64);
+  if (!grid_x_fits(tx, 256)) return TCFP_ERR_SHAPE;
+  const bool vec = al16(x);
+  if (x_fmt == TCFP_FP8_E5M2)
+    codes_t_bf16_kernel<TCFP_FP8_E5M2><<<unsigned(tx), 256, 0, st>>>(x, e_x, m, k_in, shift, mp, vec, xt);
+  else
+    codes_t_bf16_kernel<TCFP_FP8_E4M3><<<unsigned(tx), 256, 0, st>>>(x, e_x, m, k_in, shift, mp, vec, xt);
+  for (int64_t c0 = 0; c0 < n_out; c0 += rows) {
+    const int64_t n = std::min(rows, n_out - c0);
+    const int64_t tg = (mp / 64) * ((n + 63) / 64);
+    if (!grid_x_fits(tg, 256)) return TCFP_ERR_SHAPE;
+    split3_t_bf16_kernel<<<unsigned(tg), 256, 0, st>>>(g, m, n_out, c0, n, mp, gs);
+    if (hipGetLastError() != hipSuccess) return TCFP_ERR_HIP;
+    GemmArgs ga{};
+    ga.A = reinterpret_cast<const uint8_t*>(gs);
+    ga.B0 = ga.B1 = reinterpret_cast<const uint8_t*>(xt);
+    ga.M = int(n); ga.N = int(k_in); ga.K = int(6 * mp);
+    ga.lda = 6 * mp; ga.ldb = 2 * mp; ga.kwrap_b = int(2 * mp);
+    ga.s_a = inv;
+    ga.out = dw + c0 * k_in; ga.ldo = k_in;
+    int64_t kc;
+    const int64_t splits = wgrad_splits_of(6 * mp, n, k_in, &kc);
+    if (splits > 1) {
+      ga.out = part; ga.kc = int(kc); ga.split_stride = n * k_in;
+    }
+    const int rc = launch_gemm<kBF16, kBF16, true, float, 0>(ga, st);
+    if (rc != TCFP_OK) return rc;
+    if (splits > 1) {
+      const int64_t n4 = n * k_in / 4;
+      const int blocks = int(std::min<int64_t>((n4 + 255) / 256, int64_t(num_cus()) * 8));
+      splitk_reduce_kernel<<<blocks, 256, 0, st>>>(part, int(splits), n4, n * k_in, k_in, k_in,
+                                                   dw + c0 * k_in);
+      if (hipGetLastError() != hipSuccess) return TCFP_ERR_HIP;
+    }
+  }
+  return TCFP_OK;
 }

@@ -620,6 +620,34 @@ py::tuple block_linear_forward(const Tensor& x2d, const Tensor& weight, const Op
   return py::make_tuple(out, hi, lo, eh, el, aq, ae);
 }
 
+// G^T deq(X) to fp32 accuracy for any token count: per-tensor codes with their
+// inverse scale, or block codes with their exponents.
+Tensor wgrad_f32(const Tensor& grad, const Tensor& act, const OptT& inv, const OptT& act_e,
+                 int64_t bs) {
+  OnGpu g;
+  g.add(grad);
+  g.add(act);
+  g.add(inv);
+  g.add(act_e);
+  if (grad.dim() != 2 || act.dim() != 2 || grad.size(0) != act.size(0))
+    assertion("token mismatch: grad " + shape_str(grad.sizes()) + " vs act " +
+              shape_str(act.sizes()));
+  const int64_t m = grad.size(0), n = grad.size(1), k = act.size(1);
+  Tensor gr = grad.to(at::kFloat).contiguous();
+  if (!al16(gr)) gr = gr.clone();
+  const Tensor a = act.contiguous();
+  Tensor s, e;
+  if (inv) s = scalar(*inv, "scale");
+  if (act_e) e = block_scales(*act_e, m, bs > 0 ? k / bs : 0, "act_scales", at::kChar);
+  Tensor dw = g.empty({n, k}, at::kFloat);
+  const size_t nb = tcfp_wgrad_f32_workspace_bytes(m, n, k);
+  Tensor ws = g.empty({int64_t(std::max<size_t>(nb, 1))}, at::kByte);
+  check(tcfp_wgrad_f32(f32(gr), m, n, bytes(a), fmt_of(a.scalar_type()), f32(s), exps(e), k,
+                       int(bs), f32(dw), ptr(ws), nb, g.stream()),
+        "wgrad_f32");
+  return dw;
+}
+
 py::tuple block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, const OptT& act_e,
                                 const OptT& w_hi, const OptT& w_lo, const OptT& e_hi,
                                 const OptT& e_lo, int64_t bs, bool need_dx, bool need_dw,
@@ -688,6 +716,7 @@ PYBIND11_MODULE(_tcfp_host, m) {
   m.def("block_gemm", &block_gemm);
   m.def("dual_gemm_gelu_quantize", &dual_gemm_gelu_quantize);
   m.def("dual_gemm_dgelu_quantize_colsum", &dual_gemm_dgelu_quantize_colsum);
+  m.def("wgrad_f32", &wgrad_f32);
   m.def("block_linear_forward", &block_linear_forward);
   m.def("block_linear_backward", &block_linear_backward);
 }

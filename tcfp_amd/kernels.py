@@ -1137,15 +1137,15 @@ def block_scaled_wgrad(
     fp32 gradient is split into two bf16 parts and both products run as one
     bf16-MFMA GEMM; every product is exact and the split's relative
     representation error is at most 2^-17.  Token counts that are not a
-    multiple of 4 use the dequantise + fp32 matmul form.
+    multiple of 4 use three parts (:func:`wgrad_f32`).
     """
     M, N = grad.shape
     M2, Kd = act_fp8.shape
     assert M == M2, f"token mismatch: grad {tuple(grad.shape)} vs act {tuple(act_fp8.shape)}"
     dev = _hip.require_gpu(grad, act_fp8, act_scales)
-    g = grad.float().contiguous()
     if M % 4 != 0:
-        return g.t() @ block_dequantize_fp8(act_fp8, act_scales, block_size)
+        return _hip.host().wgrad_f32(grad, act_fp8, None, act_scales, block_size)
+    g = grad.float().contiguous()
     a = act_fp8.contiguous()
     e = _block_exps(act_scales, M, Kd // block_size, "act_scales")
     out = torch.empty((N, Kd), dtype=torch.float32, device=dev)
@@ -1159,6 +1159,19 @@ def block_scaled_wgrad(
         "block_wgrad",
     )
     return out
+
+
+def wgrad_f32(grad: torch.Tensor, act_fp8: torch.Tensor, act_inv: torch.Tensor) -> torch.Tensor:
+    """``grad.t() @ (act_fp8.float() * act_inv)`` in fp32 accuracy, [N, K]:
+    the per-tensor path's weight gradient where the token count is not a
+    multiple of 16 (reference ``tcfp/nn/__init__.py:553-555``, an fp32
+    matmul there).
+
+    grad [M, N], M >= 1, any count; act [M, K] FP8, K % 16 == 0; act_inv (1,)
+    fp32.  The fp32 gradient is the exact sum of three bf16 parts and the codes
+    are exact in bf16: three passes on the bf16 MFMA with fp32 accumulation.
+    """
+    return _hip.host().wgrad_f32(grad, act_fp8, act_inv, None, 0)
 
 
 def block_backward_prep(

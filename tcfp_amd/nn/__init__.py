@@ -202,6 +202,8 @@ class _TCFP12TensorCoreFunction(torch.autograd.Function):
                 grad_weight = grad_2d.t() @ saved_act.to(grad_2d.dtype)
             elif ctx.fp8_wgrad:
                 grad_weight = K.fp8_gemm_nt(grad_t, saved_act, grad_inv, act_inv)
+            elif grad_2d.dtype == torch.float32 and grad_2d.shape[0] > 0:
+                grad_weight = K.wgrad_f32(grad_2d, saved_act, act_inv)
             else:
                 grad_weight = grad_2d.t() @ (saved_act.float() * act_inv).to(grad_2d.dtype)
         if need_db and ctx.has_bias and grad_bias is None:

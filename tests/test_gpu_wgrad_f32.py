@@ -1,0 +1,84 @@
+"""The weight gradient of token counts that the FP8 and the split-bf16 products
+do not take: G^T deq(X) in fp32 accuracy as three exact bf16 passes.
+
+Bound: the fp32 product's own error.  The split is exact, so what is left is
+fp32 accumulation over the tokens: at most (3 m / 16 + a few) roundings of
+2^-24 per element, random in sign, against m for an fp32 dot; the test holds
+the relative Frobenius error to 1.2 times torch's fp32 product of the same
+operands or 2e-7, whichever is larger (2^-24 = 6e-8 is one rounding)."""
+import pytest
+import torch
+
+from tcfp_amd import kernels as K
+from tcfp_amd.nn import TCFPLinear
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(out, ref):
+    return (torch.linalg.norm(out.double() - ref) / torch.linalg.norm(ref)).item()
+
+
+# one token, the edges of the 64-row padding, ragged columns, split-K and more
+# than one chunk of dW rows (64 MiB of split gradient: m 2001 x n 6000)
+@pytest.mark.parametrize("m,n,k", [(1, 16, 16), (63, 130, 80), (65, 48, 1040), (1000, 1552, 1040),
+                                   (1001, 33, 4096), (2001, 6000, 272)])
+@pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_per_tensor(dev, m, n, k, fp8):
+    gen = torch.Generator().manual_seed(m + n)
+    g = (torch.randn(m, n, generator=gen)
+         * torch.exp2(torch.randint(-20, 20, (1, n), generator=gen))).to(dev)
+    q, inv = K.quantize_per_tensor(torch.randn(m, k, generator=gen).to(dev), fp8)
+    dw = K.wgrad_f32(g, q, inv)
+    # (per column scale of g: errors are compared row by row of dW)
+    ref = g.double().t() @ (q.double() * inv.double())
+    s = ref.norm(dim=1, keepdim=True).clamp(min=1e-300)
+    fp32 = g.t() @ (q.float() * inv)
+    err, own = _rel(dw / s, ref / s), _rel(fp32 / s, ref / s)
+    print(f"wgrad_f32 {m}x{n}x{k} {fp8}: {err:.2e} (torch fp32 {own:.2e})")
+    assert err <= max(1.2 * own, 2e-7)
+    assert torch.equal(dw, K.wgrad_f32(g, q, inv))
+
+
+@pytest.mark.parametrize("bs", [32, 64, 128])
+@pytest.mark.parametrize("m", [1, 101, 1027])
+def test_block(dev, m, bs):
+    n, k = 200, 512
+    gen = torch.Generator().manual_seed(m + bs)
+    g = torch.randn(m, n, generator=gen).to(dev)
+    x = torch.randn(m, k, generator=gen) * torch.exp2(torch.randint(-8, 8, (m, k), generator=gen))
+    q, e = K.block_quantize_fp8(x.to(dev), bs)
+    dw = K.block_scaled_wgrad(g, q, e, bs)
+    xd = K.block_dequantize_fp8(q, e, bs)
+    ref = g.double().t() @ xd.double()
+    assert _rel(dw, ref) <= max(1.2 * _rel(g.t() @ xd, ref), 2e-7)
+
+
+def test_special_gradients(dev):
+    """Non-finite and extreme gradients as the fp32 product has them: an inf
+    row stays inf, a NaN NaN, the largest and smallest normals are exact."""
+    m, n, k = 19, 64, 32
+    q = torch.ones(m, k, device=dev).to(torch.float8_e4m3fn)
+    inv = torch.ones(1, device=dev)
+    g = torch.zeros(m, n, device=dev)
+    g[3, 0] = float("inf")
+    g[4, 1] = float("nan")
+    g[5, 2] = torch.finfo(torch.float32).max
+    g[6, 3] = -1.2345678e-20
+    g[7, 4] = float("-inf")
+    dw = K.wgrad_f32(g, q, inv)
+    ref = g.t() @ q.float()
+    assert torch.equal(dw.isnan(), ref.isnan())
+    assert torch.equal(dw.nan_to_num(), ref.nan_to_num())
+
+
+def test_layer_uses_it(dev):
+    """A per-tensor layer's dW at 1000 tokens against 64 bits."""
+    torch.manual_seed(0)
+    layer = TCFPLinear(256, 320, use_tensor_cores=True).to(dev)
+    x = torch.randn(1000, 256, device=dev)
+    g = torch.randn(1000, 320, device=dev)
+    layer(x).backward(g)
+    q, inv = K.quantize_per_tensor(x)
+    ref = g.double().t() @ (q.double() * inv.double())
+    assert _rel(layer.weight.grad, ref) < 1e-6
