@@ -616,6 +616,14 @@ int tcfp_block_dual_gemm_dx_bf16(const uint16_t* g_deq, const uint8_t* w_hi, con
                                  int64_t d_in, int block, float* dx, void* workspace,
                                  size_t workspace_bytes, void* stream);
 
+/* The same with dX in fp32 or bf16 (dx_dtype; bf16: the fp32 result rounded
+ * to nearest even, what autograd makes of an fp32 gradient of a bf16 input). */
+int tcfp_block_dual_gemm_dx_bf16_to(const uint16_t* g_deq, const uint8_t* w_hi,
+                                    const uint8_t* w_lo, const int8_t* e_hi, const int8_t* e_lo,
+                                    int64_t m, int64_t d_out, int64_t d_in, int block, void* dx,
+                                    int dx_dtype, void* workspace, size_t workspace_bytes,
+                                    void* stream);
+
 /* tcfp_block_wgrad with the gradient already split and transposed
  * (g_split_t [n_out, 2m] from tcfp_block_grad_prep with split_lo 1): same
  * result bit for bit.  With split_lo 0, g_split_t is [n_out, m] (bf16(g)

@@ -131,6 +131,9 @@ _SIGNATURES = {
     "tcfp_block_dual_gemm_dx_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64,
                                      _i64, _i64, _i32, _c_void_p, _c_void_p, ctypes.c_size_t,
                                      _c_void_p],
+    "tcfp_block_dual_gemm_dx_bf16_to": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                                        _i64, _i64, _i64, _i32, _c_void_p, _i32, _c_void_p,
+                                        ctypes.c_size_t, _c_void_p],
     "tcfp_block_dual_gemm_dx_bf16_workspace_bytes": [_i64, _i64],
     "tcfp_wgrad_f32_workspace_bytes": [_i64, _i64, _i64],
     "tcfp_wgrad_f32": [_c_void_p, _i64, _i64, _c_void_p, _i32, _c_void_p, _c_void_p, _i64, _i32,

@@ -3140,9 +3140,9 @@ int64_t dgrad_chunk(int64_t d_out, int64_t d_in) { return chunk_cols(4 * d_out, 
 
 // Per chunk of dx columns [c0, c0 + n): W_hi^T, W_lo^T rows c0.. dequantised
 // into bf16 (one launch), then the bf16 dual GEMM A = G [m, d_out] x
-// B = W^T [n, d_out] (K counts bytes) into dx[:, c0 ..] (fp32, ld d_in).
+// B = W^T [n, d_out] (K counts bytes) into dx[:, c0 ..] (fp32 or bf16, ld d_in).
 int dgrad_bf16(const uint16_t* gd, const uint8_t* w_hi, const uint8_t* w_lo, const int8_t* e_hi,
-               const int8_t* e_lo, int64_t m, int64_t d_out, int64_t d_in, int shift, float* dx,
+               const int8_t* e_lo, int64_t m, int64_t d_out, int64_t d_in, int shift, void* dx, int dx_dtype,
                uint16_t* wth, uint16_t* wtl, hipStream_t st) {
   const int64_t cw = dgrad_chunk(d_out, d_in);
   for (int64_t c0 = 0; c0 < d_in; c0 += cw) {
@@ -3161,9 +3161,17 @@ int dgrad_bf16(const uint16_t* gd, const uint8_t* w_hi, const uint8_t* w_lo, con
     ga.B1 = reinterpret_cast<const uint8_t*>(w_lo ? wtl : wth);
     ga.M = int(m); ga.N = int(n); ga.K = int(2 * d_out);
     ga.lda = 2 * d_out; ga.ldb = 2 * d_out;
-    ga.out = dx + c0; ga.ldo = d_in;
-    const int rc = w_lo ? launch_gemm<kBF16, kBF16, false, float, 0>(ga, st)
-                        : launch_gemm<kBF16, kBF16, true, float, 0>(ga, st);
+    ga.ldo = d_in;
+    int rc;
+    if (dx_dtype == TCFP_DTYPE_BF16) {
+      ga.out = static_cast<uint16_t*>(dx) + c0;
+      rc = w_lo ? launch_gemm<kBF16, kBF16, false, uint16_t, 0>(ga, st)
+                : launch_gemm<kBF16, kBF16, true, uint16_t, 0>(ga, st);
+    } else {
+      ga.out = static_cast<float*>(dx) + c0;
+      rc = w_lo ? launch_gemm<kBF16, kBF16, false, float, 0>(ga, st)
+                : launch_gemm<kBF16, kBF16, true, float, 0>(ga, st);
+    }
     if (rc != TCFP_OK) return rc;
   }
   return TCFP_OK;
@@ -3214,7 +3222,8 @@ extern "C" int tcfp_block_dual_gemm_dx(const uint8_t* g, int g_fmt, const int8_t
       dequant_rows_bf16_kernel<TCFP_FP8_E4M3><<<unsigned(gr), 256, 0, st>>>(g, e_g, m, d_out, shift, 0, gd);
     if (hipGetLastError() != hipSuccess) return TCFP_ERR_HIP;
   }
-  return dgrad_bf16(gd, w_hi, w_lo, e_hi, e_lo, m, d_out, d_in, shift, dx, wth, wtl, st);
+  return dgrad_bf16(gd, w_hi, w_lo, e_hi, e_lo, m, d_out, d_in, shift, dx, TCFP_DTYPE_F32, wth,
+                    wtl, st);
 }
 
 extern "C" size_t tcfp_block_dual_gemm_dx_bf16_workspace_bytes(int64_t d_out, int64_t d_in) {
@@ -3222,14 +3231,15 @@ extern "C" size_t tcfp_block_dual_gemm_dx_bf16_workspace_bytes(int64_t d_out, in
   return 2 * dgrad_copy_bytes(d_out, d_in);
 }
 
-extern "C" int tcfp_block_dual_gemm_dx_bf16(const uint16_t* g_deq, const uint8_t* w_hi,
+extern "C" int tcfp_block_dual_gemm_dx_bf16_to(const uint16_t* g_deq, const uint8_t* w_hi,
                                             const uint8_t* w_lo, const int8_t* e_hi,
                                             const int8_t* e_lo, int64_t m, int64_t d_out,
-                                            int64_t d_in, int block, float* dx, void* workspace,
+                                            int64_t d_in, int block, void* dx, int dx_dtype, void* workspace,
                                             size_t workspace_bytes, void* stream) {
   if (m < 0 || d_out < 0 || d_in < 0 || m > INT32_MAX || d_in > INT32_MAX ||
       2 * d_out > INT32_MAX)
     return TCFP_ERR_SHAPE;
+  if (dx_dtype != TCFP_DTYPE_F32 && dx_dtype != TCFP_DTYPE_BF16) return TCFP_ERR_DTYPE;
   if (block != 32 && block != 64 && block != 128) return TCFP_ERR_SHAPE;
   if (d_out % block != 0 || d_in % block != 0) return TCFP_ERR_SHAPE;
   if (!g_deq || !w_hi || !e_hi || (w_lo && !e_lo) || !dx) return TCFP_ERR_SHAPE;
@@ -3241,8 +3251,17 @@ extern "C" int tcfp_block_dual_gemm_dx_bf16(const uint16_t* g_deq, const uint8_t
   uint8_t* ws = static_cast<uint8_t*>(workspace);
   uint16_t* wth = reinterpret_cast<uint16_t*>(ws);
   uint16_t* wtl = reinterpret_cast<uint16_t*>(ws + dgrad_copy_bytes(d_out, d_in));
-  return dgrad_bf16(g_deq, w_hi, w_lo, e_hi, e_lo, m, d_out, d_in, shift, dx, wth, wtl,
+  return dgrad_bf16(g_deq, w_hi, w_lo, e_hi, e_lo, m, d_out, d_in, shift, dx, dx_dtype, wth, wtl,
                     static_cast<hipStream_t>(stream));
+}
+
+extern "C" int tcfp_block_dual_gemm_dx_bf16(const uint16_t* g_deq, const uint8_t* w_hi,
+                                            const uint8_t* w_lo, const int8_t* e_hi,
+                                            const int8_t* e_lo, int64_t m, int64_t d_out,
+                                            int64_t d_in, int block, float* dx, void* workspace,
+                                            size_t workspace_bytes, void* stream) {
+  return tcfp_block_dual_gemm_dx_bf16_to(g_deq, w_hi, w_lo, e_hi, e_lo, m, d_out, d_in, block, dx,
+                                         TCFP_DTYPE_F32, workspace, workspace_bytes, stream);
 }
 
 namespace {

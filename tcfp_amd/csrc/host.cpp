@@ -651,7 +651,7 @@ Tensor wgrad_f32(const Tensor& grad, const Tensor& act, const OptT& inv, const O
 py::tuple block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, const OptT& act_e,
                                 const OptT& w_hi, const OptT& w_lo, const OptT& e_hi,
                                 const OptT& e_lo, int64_t bs, bool need_dx, bool need_dw,
-                                bool want_db, bool split_lo) {
+                                bool want_db, bool split_lo, at::ScalarType dx_dtype) {
   const int64_t M = grad_2d.size(0), N = grad_2d.size(1);
   const int64_t K = need_dx ? w_hi->size(1) : need_dw ? act_fp8->size(1) : 0;
   OnGpu g;
@@ -689,12 +689,12 @@ py::tuple block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, cons
   }
   g_split.reset();
   if (need_dx) {
-    dx = g.empty({M, K}, at::kFloat);
+    dx = g.empty({M, K}, dx_dtype);
     const size_t n = tcfp_block_dual_gemm_dx_bf16_workspace_bytes(N, K);
     Tensor ws = scratch(n);
-    check(tcfp_block_dual_gemm_dx_bf16(ptr<uint16_t>(g_deq), bytes(*w_hi), bytes(opt(w_lo)),
-                                       exps(*e_hi), exps(opt(e_lo)), M, N, K, int(bs), f32(dx),
-                                       ptr(ws), n, st),
+    check(tcfp_block_dual_gemm_dx_bf16_to(ptr<uint16_t>(g_deq), bytes(*w_hi), bytes(opt(w_lo)),
+                                          exps(*e_hi), exps(opt(e_lo)), M, N, K, int(bs), ptr(dx),
+                                          out_dtype_of(dx_dtype), ptr(ws), n, st),
           "block_dgrad_from_prep");
   }
   auto ret = [](const Tensor& t) -> py::object {

@@ -1224,7 +1224,7 @@ def block_backward_prep(
 
 
 def block_linear_backward(grad_2d, act_fp8, act_e, w_hi, w_lo, e_hi, e_lo, block_size,
-                          need_dx, need_dw, want_db, split_lo=True):
+                          need_dx, need_dw, want_db, split_lo=True, dx_dtype=torch.float32):
     """The launches of a block-scaled TCFP layer's default backward, as
     :func:`block_backward_prep`, :func:`block_wgrad_from_prep` and
     :func:`block_dgrad_from_prep` run them, with the same results bit for
@@ -1236,10 +1236,12 @@ def block_linear_backward(grad_2d, act_fp8, act_e, w_hi, w_lo, e_hi, e_lo, block
     ``grad_2d`` [M, D_out]; ``act_fp8`` / ``act_e`` the forward's activation
     codes and exponents (``need_dw``; M % 4 == 0, and M % 64 == 0 without
     ``split_lo``); ``w_hi`` .. ``e_lo`` the forward's weight operands
-    (``need_dx``).  Returns ``(dx fp32 [M, D_in], dw fp32 [D_out, D_in],
-    db fp32 [D_out])``, None where not requested."""
+    (``need_dx``).  Returns ``(dx [M, D_in] in dx_dtype (fp32, or bf16: the
+    fp32 values rounded), dw fp32 [D_out, D_in], db fp32 [D_out])``, None where
+    not requested."""
     return _hip.host().block_linear_backward(grad_2d, act_fp8, act_e, w_hi, w_lo, e_hi, e_lo,
-                                             block_size, need_dx, need_dw, want_db, split_lo)
+                                             block_size, need_dx, need_dw, want_db, split_lo,
+                                             dx_dtype)
 
 
 def block_dgrad_from_prep(g_deq, w_hi_fp8, w_lo_fp8, w_hi_scales, w_lo_scales, block_size):

@@ -64,6 +64,12 @@ def _for_inference(*tensors):
     return tuple(t.detach() if t is not None and t.requires_grad else t for t in tensors)
 
 
+def _grad_dtype(x: torch.Tensor) -> torch.dtype:
+    """The type dX is written in: x's own where the GEMMs write it (autograd
+    would cast an fp32 gradient to it anyway, with the same rounding)."""
+    return torch.bfloat16 if x.dtype == torch.bfloat16 else torch.float32
+
+
 def _ef_buffer(state: ErrorFeedbackState | None, name: str, weight: torch.Tensor):
     if state is None:
         return None
@@ -150,6 +156,7 @@ class _TCFP12TensorCoreFunction(torch.autograd.Function):
         # 8. save for backward
         ctx.hp_grad_weight = hp_grad_weight
         ctx.input_shape = input_shape
+        ctx.dx_dtype = _grad_dtype(input)
         ctx.has_bias = bias is not None
         ctx.abd = abd
         ctx.fp8_wgrad = fp8_wgrad
@@ -192,10 +199,10 @@ class _TCFP12TensorCoreFunction(torch.autograd.Function):
                 (grad_fp8, grad_inv), grad_t = res, None
             if need_dx:
                 if ctx.abd:
-                    gi = K.fp8_gemm_nt(grad_fp8, w_hi_t, grad_inv, inv_hi)
+                    gi = K.fp8_gemm_nt(grad_fp8, w_hi_t, grad_inv, inv_hi, out_dtype=ctx.dx_dtype)
                 else:
                     gi = K._dual_gemm(grad_fp8, w_hi_t, w_lo_t, grad_inv, inv_hi, inv_lo,
-                                      None, torch.float32)
+                                      None, ctx.dx_dtype)
                 grad_input = gi.reshape(ctx.input_shape)
         if need_dw:
             if ctx.hp_grad_weight:
@@ -291,6 +298,7 @@ class _TCFP12BlockScaledFunction(torch.autograd.Function):
 
         ctx.hp_grad_weight = hp_grad_weight
         ctx.input_shape = input_shape
+        ctx.dx_dtype = _grad_dtype(input)
         ctx.has_bias = bias is not None
         ctx.bs = bs
         ctx.abd = abd
@@ -333,7 +341,7 @@ class _TCFP12BlockScaledFunction(torch.autograd.Function):
             # in one host call (the same launches as below)
             dx, dw, db = K.block_linear_backward(
                 grad_2d, saved_act, act_scales, w_hi, w_lo, sh, sl, bs, need_dx, need_dw,
-                want_db, split_lo=split_lo)
+                want_db, split_lo=split_lo, dx_dtype=ctx.dx_dtype)
             if dx is not None:
                 grad_input = dx.reshape(ctx.input_shape)
             if dw is not None:
@@ -635,6 +643,7 @@ class _TCFP12FusedMLPFunction(torch.autograd.Function):
         out = K.fused_dual_gemm_forward(a2, w2_hi, w2_lo, a2_inv, ih2, il2, bias=b2)
 
         ctx.input_shape = input_shape
+        ctx.dx_dtype = _grad_dtype(x)
         ctx.has_b1, ctx.has_b2 = b1 is not None, b2 is not None
         ctx.save_for_backward(
             a1_t, a1_inv, w1_hi_t, w1_lo_t, ih1, il1,
@@ -686,7 +695,7 @@ class _TCFP12FusedMLPFunction(torch.autograd.Function):
                 db1 = res[-1]
             if need_dx:
                 grad_x = K._dual_gemm(q1, w1_hi_t, w1_lo_t, g1_inv, ih1, il1, None,
-                                      torch.float32).reshape(ctx.input_shape)
+                                      ctx.dx_dtype).reshape(ctx.input_shape)
             if need_dw1:
                 dw1 = K.fp8_gemm_nt(q1_t, a1_t, g1_inv, a1_inv)
         return (grad_x, dw1, db1, dw2, db2) + (None,) * 6

@@ -166,3 +166,32 @@ def test_mid_tile_matches_small_tile(dev, policy, m, n, k, bs, od):
     assert any("4, 128, 128, " in s for s in names), names
     assert torch.equal(out, small)
     assert _rel(out, ref + bias.double()) < (1e-4 if od == torch.float32 else 3e-3)
+
+
+# every tile a dgrad may take: the weight stream, one round of the small tile,
+# the 128 x 128 tile, the large one, the persistent one with eight and four waves
+@pytest.mark.parametrize("m,n,k", [(40, 520, 256), (300, 512, 400), (1000, 4096, 1024),
+                                   (8192, 1024, 384), (4096, 4096, 256), (2048, 4608, 8192)])
+def test_bf16_gradient_is_the_rounded_fp32_one(dev, m, n, k):
+    g = torch.Generator().manual_seed(m + k)
+    a, sa = K.quantize_per_tensor(torch.randn(m, k, generator=g).to(dev), E5M2)
+    hi, lo, ih, il = K.dual_quantize_per_tensor(torch.randn(n, k, generator=g).to(dev))
+    f32 = K._dual_gemm(a, hi, lo, sa, ih, il, None, torch.float32)
+    assert torch.equal(K._dual_gemm(a, hi, lo, sa, ih, il, None, torch.bfloat16), f32.bfloat16())
+
+
+@pytest.mark.parametrize("m,n,k", [(100, 128, 192), (4096, 256, 1024), (2048, 4096, 8192)])
+def test_block_backward_bf16_gradient(dev, m, n, k):
+    """block_linear_backward's dX in bf16 is its fp32 dX rounded (with W_lo, and
+    W_hi alone), dW and db the same."""
+    g = torch.Generator().manual_seed(m + k)
+    gr = torch.randn(m, n, generator=g).to(dev)
+    out = K.block_linear_forward(torch.randn(m, k, generator=g).bfloat16().to(dev),
+                                 (torch.randn(n, k, generator=g) * 0.02).to(dev), None, 64)
+    _, hi, lo, eh, el, aq, ae = out
+    for lo_, el_ in ((lo, el), (None, None)):
+        ref = K.block_linear_backward(gr, aq, ae, hi, lo_, eh, el_, 64, True, True, True)
+        got = K.block_linear_backward(gr, aq, ae, hi, lo_, eh, el_, 64, True, True, True,
+                                      dx_dtype=torch.bfloat16)
+        assert torch.equal(got[0], ref[0].bfloat16())
+        assert torch.equal(got[1], ref[1]) and torch.equal(got[2], ref[2])
