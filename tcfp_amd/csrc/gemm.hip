@@ -358,7 +358,9 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // ---- tile mapping (XCD-aware, grouped) ----
   const int T = g.tiles_m * g.tiles_n;
   int l = blockIdx.x;
-  if ((T & 7) == 0) l = (l & 7) * (T >> 3) + (l >> 3);
+  // (each XCD a run of adjacent tiles, the first T % 8 of them one more; T %
+  // 8 != 0 in plain order ran 2256 x 12000 x 3008 in 178.8 us against 162.1)
+  l = (l & 7) * (T >> 3) + min(l & 7, T & 7) + (l >> 3);
   // 4 tile-rows per group: the 32 workgroups an XCD runs at once share 4
   // A panels (8 wide groups re-read a large A once per 4 column tiles: the
   // 16384 x 4096 x 16384 split-bf16 wgrad ran 1.80 ms grouped by 8 against
@@ -1296,10 +1298,20 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
 //    stores (loads and stores retire in issue order under vmcnt), so the
 //    output drains to memory while the next tile computes.
 // The per-stage schedule is the large tile's of gemm_nt_dma_kernel.
-// Launched only for full tiles (M % 256 == 0, N % 128 == 0, K % 128 == 0,
-// K > 128: two stages at least) and a 16-byte aligned output with
-// ldo % 8 == 0: every wave then issues exactly NST store instructions per
-// tile, which the vmcnt accounting above relies on, and no stage is partial.
+// Launched with two K stages at least (K > 128) and a 16-byte aligned output
+// with whole 16-byte vectors per row: every wave then issues exactly NST
+// store instructions per tile, which the vmcnt accounting above relies on.
+// EPI 0 - 2 take full tiles only (M % 256 == 0, N % 128 == 0, K % 128 == 0),
+// EPI 3 (RAG) any M, N and K % 16 == 0: rows past the matrix are beyond the
+// tile's descriptors and read as zeros, the last stage's chunks past K are
+// sent out of range, and the stores go through a buffer descriptor that
+// drops what lies outside, so that an edge tile issues as many as a full
+// one.  Against one workgroup per tile, which every ragged size took before
+// (us, one process): 4112 x 4112 x 256 bf16 33.6 -> 20.8, 16384 x 4112 x 512
+// bf16 126.6 -> 82.1, 8000 x 4000 x 1040 fp32 98.2 -> 86.4, 4000 x 4096 x
+// 4096 bf16 112.2 -> 103.8 and block 64 128.2 -> 113.1, 8176 x 8176 x 4096
+// block 32 508 -> 442, 8000 x 4096 x 8192 fp32 410 -> 400 (power cap from
+// there on).  Full tiles keep the plain variant, whose offsets are constants.
 //
 // fp32 output (OutT = float) skips the LDS staging: each lane stores its
 // accumulator rows as 16-byte vectors straight from registers (16 stores per
@@ -1320,12 +1332,14 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
 // 256 x 64 slots' do.
 template <int AF, int BF, typename OutT, int EPI = 0, int SCALE = 0, int ND = 8, int BNT = 128,
           bool SPL = false>
-__global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_persist_kernel(
-    GemmArgs g) {
+TCFP_DEV void persist_tiles(const GemmArgs g) {
   constexpr bool F32OUT = std::is_same<OutT, float>::value;
-  static_assert(EPI == 0 || F32OUT, "GELU epilogues write fp32");
-  static_assert(SCALE == 0 || (SCALE == 1 && EPI == 0), "block exponents: plain epilogue only");
+  constexpr bool RAG = EPI == 3;
+  constexpr bool PLAIN = EPI == 0 || RAG;
+  static_assert(PLAIN || F32OUT, "GELU epilogues write fp32");
+  static_assert(SCALE == 0 || (SCALE == 1 && PLAIN), "block exponents: plain epilogue only");
   static_assert(!SPL || (EPI == 0 && F32OUT), "single GEMM: fp32, plain epilogue");
+  static_assert(!RAG || (ND == 8 && BNT == 128), "ragged sizes: the eight-wave dual tile");
   constexpr int NACC = (SCALE == 1 && !SPL) ? 1 : 2;
   constexpr int NSL = SPL ? 2 : 1;  // output column blocks per tile
   // ROLL (single GEMM, 256 x 128 slots: a 256 x 256 output tile): the two
@@ -1432,7 +1446,7 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
   const uint8_t* const src_base = region == 0 ? g.A : (region == 1 ? g.B0 : g.B1);
   const int64_t ld = region == 0 ? g.lda : g.ldb;
   const int region_rows = region == 0 ? BM : BN;
-  const uint32_t nrec = uint32_t(int64_t(region_rows - 1) * ld + K);  // full tiles only
+  const uint32_t nrec = uint32_t(int64_t(region_rows - 1) * ld + K);  // (of a full tile)
   const int chunk0 = (lane & 7) ^ swz(lane >> 3);
   const int chunk1 = (lane & 7) ^ swz(8 + (lane >> 3));
   // byte offsets of this lane's row within a tile for even / odd DMA
@@ -1444,12 +1458,15 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
   const uint32_t row8 = uint32_t(8 * ld);
   const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((TCFP_LDS uint8_t*)lds));
   const uint32_t lds_base = lds0 + uint32_t(srow0) * kRowB;
-  const int nt = K / kSK;
+  const int nt = RAG ? (K + kSK - 1) / kSK : K / kSK;
+  // RAG: this lane's chunks of the last stage past K
+  const bool past0 = RAG && (nt - 1) * kSK + chunk0 * 16 >= K;
+  const bool past1 = RAG && (nt - 1) * kSK + chunk1 * 16 >= K;
 
   // tile `it` of this workgroup -> (m0, n0)
   auto tile_of = [&](int it, int& m0, int& n0) {
     int l = int(blockIdx.x) + it * int(gridDim.x);
-    if ((T & 7) == 0) l = (l & 7) * (T >> 3) + (l >> 3);
+    l = (l & 7) * (T >> 3) + min(l & 7, T & 7) + (l >> 3);
     // groups of 4 tile-rows, as in gemm_nt_dma_kernel (A/B on two boxes
     // against 8: 4096^3 95.4 -> 93.9 us, 8192 x 4096 x 1024 fp32 out
     // 71.2 -> 67.5 us, 8192 x 16384 x 4096 block 1018 -> 952 us; 8192 x
@@ -1462,6 +1479,11 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
     n0 = ((l % per_group) / gm) * (NSL * BN);
   };
   auto src_of = [&](int m0, int n0) {
+    if constexpr (RAG) {
+      const int left = min(region_rows, region == 0 ? M - m0 : N - n0);
+      return make_rsrc(src_base + int64_t(region == 0 ? m0 : n0) * ld,
+                       uint32_t(int64_t(left - 1) * ld + K));
+    }
     return make_rsrc(src_base + int64_t(region == 0 ? m0 : n0) * ld, nrec);
   };
   // DMA of stage t of the tile whose operand rows `rs` describes into buffer b
@@ -1474,6 +1496,19 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
     // DMA before it)
     uint32_t vb0 = voff0, vb1 = voff1;
     if constexpr (W4) asm volatile("" : "+v"(vb0), "+v"(vb1));
+    if constexpr (RAG) {
+      // (chunks past K; stepped in two registers, see W4)
+      vb0 = t == nt - 1 && past0 ? kOob : vb0;
+      vb1 = t == nt - 1 && past1 ? kOob : vb1 + row8;
+#pragma unroll
+      for (int i = 0; i < DI; ++i) {
+        uint32_t& vb = (i & 1) ? vb1 : vb0;
+        asm volatile("" : "+v"(vb));
+        dma16(rs, vb, soff, dst + i * 1024);
+        vb += 2 * row8;
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < DI; ++i)
       dma16(rs, ((i & 1) ? vb1 : vb0) + uint32_t(i) * row8, soff, dst + i * 1024);
@@ -1560,8 +1595,16 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
     if constexpr (SCALE == 1) {
       // waves 2 (t % (ND / 2)) and 2 (t % (ND / 2)) + 1 (all of them DMA waves)
       if ((wave >> 1) == t % (ND / 2)) {
-        const int8_t* src =
-            ebase + (int64_t(t) * kbs + ekb) * eld + (ereg == 0 ? mt : ntl) + erow;
+        int64_t kb = int64_t(t) * kbs + ekb;
+        int row = (ereg == 0 ? mt : ntl) + erow;
+        if constexpr (RAG) {
+          // (16-row chunks lie inside the matrix or outside, M and N being
+          // multiples of 16: one outside, or a K block past K, re-reads a
+          // valid one beside zero operands)
+          kb = min(kb, int64_t(K >> bsh) - 1);
+          if (row >= int(eld)) row = 0;
+        }
+        const int8_t* src = ebase + kb * eld + row;
         gdma16(src, exp_lds0 + uint32_t(b) * kExpStage + uint32_t(wave & 1) * 1024u);
       }
     }
@@ -1713,7 +1756,7 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
       const bool bias_stage =
           kBiasLds && g.bias != nullptr && t == (nt > 2 ? nt - 2 : 0) && tid < NSL * BN;
       float bv = 0.0f;
-      if (bias_stage) bv = g.bias[n0 + tid];
+      if (bias_stage) bv = g.bias[RAG ? min(n0 + tid, N - 1) : n0 + tid];
       if constexpr (W4) {
         // One wave per SIMD: nothing else hides a stall, so the stage is
         // one fixed sequence.  Sub-step 0's first half with the fragments
@@ -1976,6 +2019,17 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
         read_frags(f0, sb ^ 1, 0);
       } else {
         // (SPL: output column block sl of the tile from accumulator set sl)
+        // (RAG: rows past the matrix lie beyond the descriptor, columns past
+        // it are sent there; the lane's offset is laundered, as it would
+        // otherwise be kept across the K loop, where no register is free)
+        const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<float*>(out) + int64_t(m0) * g.ldo + n0, 0,
+            int(RAG ? uint32_t(min(BM, M - m0)) * ldo_b : 0u), 0x00020000);
+        int lane_o = lane;
+        if constexpr (RAG) asm volatile("" : "+v"(lane_o));
+        const uint32_t vlane = uint32_t(wm * TMW + (lane_o & 31)) * ldo_b +
+                               uint32_t(wn * TNW + (lane_o >> 5) * 4) * 4u;
+        const int ncol = N - nb - (lane_o >> 5) * 4;
 #pragma unroll
         for (int sl = 0; sl < NSL; ++sl)
 #pragma unroll
@@ -1986,6 +2040,9 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
             for (int gq = 0; gq < 4; ++gq) {
               const int row = i * 32 + lr, col = sl * BN + j * 32 + gq * 8 + lg * 4;
               const int64_t o = int64_t(m0 + wm * TMW + row) * g.ldo + nb + col;
+              const uint32_t vo = j * 32 + gq * 8 < ncol
+                                      ? vlane + uint32_t(i * 32) * ldo_b + uint32_t(j * 32 + gq * 8) * 4u
+                                      : kOob;
               float v[4];
 #pragma unroll
               for (int q = 0; q < 4; ++q) {
@@ -2004,10 +2061,19 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
                   v[3] += b4.w;
                 } else {
 #pragma unroll
-                  for (int q = 0; q < 4; ++q) v[q] += g.bias[nb + col + q];
+                  for (int q = 0; q < 4; ++q)
+                    v[q] += g.bias[RAG ? N - max(ncol - (j * 32 + gq * 8), 4) + q : nb + col + q];
                 }
               }
-              store4<float>(reinterpret_cast<float*>(out) + o, v[0], v[1], v[2], v[3]);
+              if constexpr (RAG) {
+                typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+                __builtin_amdgcn_raw_buffer_store_b128(
+                    u4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]),
+                       __float_as_uint(v[3])},
+                    orsrc, vo, 0, 0);
+              } else {
+                store4<float>(reinterpret_cast<float*>(out) + o, v[0], v[1], v[2], v[3]);
+              }
               if constexpr (EPI == 1) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
@@ -2056,7 +2122,8 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
               v[3] += b4.w;
             } else {
 #pragma unroll
-              for (int q = 0; q < 4; ++q) v[q] += g.bias[nb + col + q];
+              for (int q = 0; q < 4; ++q)
+                v[q] += g.bias[RAG ? min(nb + col, N - 4) + q : nb + col + q];
             }
           }
           const int byte = col * 2;
@@ -2088,8 +2155,19 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
       issue(nxt, 1, sb);
     }
     __builtin_amdgcn_sched_barrier(0);
+    const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(
+        out + int64_t(m0) * g.ldo + n0, 0,
+        int(RAG ? uint32_t(min(BM, M - m0)) * uint32_t(g.ldo) * 2u : 0u), 0x00020000);
     auto put = [&](int s, const uint4& d) {
       const int row = s * RPI + lane_e / CPR, cl = lane_e % CPR;
+      if constexpr (RAG) {
+        const uint32_t vo = nb + cl * 8 < N ? (uint32_t(wm * TMW + row) * uint32_t(g.ldo) +
+                                               uint32_t(wn * TNW + cl * 8)) * 2u
+                                            : kOob;
+        typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+        __builtin_amdgcn_raw_buffer_store_b128(u4{d.x, d.y, d.z, d.w}, orsrc, vo, 0, 0);
+        return;
+      }
       OutT* o = out + int64_t(m0 + wm * TMW + row) * g.ldo + nb + cl * 8;
       *reinterpret_cast<uint4*>(o) = d;
     };
@@ -2106,7 +2184,7 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
     m0 = m1;
     n0 = n1;
   }
-  if constexpr (EPI != 0) {
+  if constexpr (!PLAIN) {
     // the workgroup's partials (no DMA is in flight after the last tile; the
     // barrier retires every wave's last LDS reads before the operand
     // buffer takes the per-wave maxima)
@@ -2138,6 +2216,19 @@ __global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_
       }
     }
   }
+}
+
+template <int AF, int BF, typename OutT, int EPI = 0, int SCALE = 0, int ND = 8, int BNT = 128,
+          bool SPL = false>
+__global__ __launch_bounds__(BNT == 128 && ND == 4 ? 256 : 512, 1) void gemm_nt_persist_kernel(
+    GemmArgs g) {
+  persist_tiles<AF, BF, OutT, EPI, SCALE, ND, BNT, SPL>(g);
+}
+
+// The same on any sizes (see EPI 3).
+template <int AF, int BF, typename OutT, int SCALE>
+__global__ __launch_bounds__(512, 1) void gemm_nt_ragged_kernel(GemmArgs g) {
+  persist_tiles<AF, BF, OutT, 3, SCALE, 8, 128, false>(g);
 }
 
 // ---------------------------------------------------------------------------
@@ -2347,6 +2438,25 @@ bool persist_eligible(const GemmArgs& ga) {
   return int64_t(ga.M / 256) * (ga.N / 128) > num_cus();
 }
 
+// The persistent launch on any sizes (EPI 3): more tiles than CUs (fewer run
+// in one round, where nothing follows a tile that its epilogue could overlap
+// with), two K stages at least, whole 16-byte output vectors, exponent chunks
+// inside or outside the matrix as a whole.
+bool persist_ragged_eligible(const GemmArgs& ga, bool f32out, int scale) {
+  if (g_tile_policy != 0 && g_tile_policy != 1) return false;
+  const int vec = f32out ? 4 : 8;
+  if (ga.K % 16 != 0 || ga.K <= kSK || ga.N % vec != 0 || ga.ldo % vec != 0 || !al16(ga.out))
+    return false;
+  if (ga.kwrap_b || (ga.kc > 0 && ga.kc < ga.K)) return false;
+  if (int64_t(256) * ga.lda + ga.K >= kMaxSpan || int64_t(128) * ga.ldb + ga.K >= kMaxSpan ||
+      int64_t(256) * ga.ldo * (f32out ? 4 : 2) >= kMaxSpan)
+    return false;
+  if (scale == 1 && (ga.M % 16 != 0 || ga.N % 16 != 0 ||
+                     int64_t(ga.K >> ga.bs_shift) * std::max(ga.M, ga.N) >= int64_t(INT32_MAX)))
+    return false;
+  return int64_t((ga.M + 255) / 256) * ((ga.N + 127) / 128) > num_cus();
+}
+
 // The persistent kernel DMAs each stage's block exponents into LDS as
 // 16-byte chunks of the exponent arrays: their bases must be 16-byte aligned
 // (rows and columns of its full tiles are multiples of 64).
@@ -2544,6 +2654,10 @@ int launch_gemm(GemmArgs ga, hipStream_t st) {
             }
           }
           gemm_nt_persist_kernel<AF, BF, OutT, 0, SCALE><<<unsigned(num_cus()), 512, 0, st>>>(ga);
+        } else if (persist_ragged_eligible(ga, std::is_same<OutT, float>::value, SCALE) &&
+                   (SCALE == 0 || exps_al16(ga))) {
+          persist = true;
+          gemm_nt_ragged_kernel<AF, BF, OutT, SCALE><<<unsigned(num_cus()), 512, 0, st>>>(ga);
         }
       }
       if (!persist)

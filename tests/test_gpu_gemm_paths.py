@@ -195,3 +195,45 @@ def test_block_backward_bf16_gradient(dev, m, n, k):
                                       dx_dtype=torch.bfloat16)
         assert torch.equal(got[0], ref[0].bfloat16())
         assert torch.equal(got[1], ref[1]) and torch.equal(got[2], ref[2])
+
+
+# more 256 x 128 tiles than CUs with partial tiles at the right, below and
+# both, a partial last stage (K % 128 != 0) and none, tile counts that the
+# eight XCDs share unevenly, outputs narrower than a tile, exponent chunks
+# outside the matrix and exponent blocks past K
+RAGGED = [(4097, 4104, 144, 0), (4000, 4352, 1024, 0), (4096, 4096 + 8, 400, 0),
+          (65793, 8, 272, 0), (260, 17000, 400, 0), (4112, 4112, 288, 32), (4352, 4112, 320, 64),
+          (65552, 16, 384, 128), (4336, 4096, 416, 32)]
+
+
+@pytest.mark.parametrize("od", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,bs", RAGGED)
+def test_ragged_persistent_tiles_match_small_tile(dev, m, n, k, bs, od):
+    """Back-to-back tiles of ragged matrices give the bits of the 128 x 64
+    tile (the same products in the same order of K), with and without a bias."""
+    g = torch.Generator().manual_seed(m + n + k + bs)
+    x = torch.randn(m, k, generator=g).to(dev)
+    w = (torch.randn(n, k, generator=g)
+         * torch.exp2(torch.randint(-9, 9, (n, 1), generator=g))).to(dev)
+    for bias in (None, torch.randn(n, generator=g).to(dev)):
+        if bs:
+            a, ea = K.block_quantize_fp8(x, bs, E5M2)
+            hi, lo, eh, el = K.fused_dual_quantize_fp8(w, bs)
+
+            def run():
+                return K.fused_block_scaled_dual_gemm_forward(a, hi, lo, ea, eh, el, bs,
+                                                              bias=bias, out_dtype=od)
+        else:
+            a, sa = K.quantize_per_tensor(x)
+            hi, lo, ih, il = K.dual_quantize_per_tensor(w)
+
+            def run():
+                return K.fused_dual_gemm_forward(a, hi, lo, sa, ih, il, bias=bias, out_dtype=od)
+        names = _kernel_names(run)
+        assert any("gemm_nt_ragged_kernel" in s for s in names), names
+        out = run()
+        try:
+            K.set_gemm_tile_policy("small")
+            assert torch.equal(out, run())
+        finally:
+            K.set_gemm_tile_policy("auto")
