@@ -358,9 +358,10 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   // ---- tile mapping (XCD-aware, grouped) ----
   const int T = g.tiles_m * g.tiles_n;
   int l = blockIdx.x;
-  // (each XCD a run of adjacent tiles, the first T % 8 of them one more; T %
-  // 8 != 0 in plain order ran 2256 x 12000 x 3008 in 178.8 us against 162.1)
-  l = (l & 7) * (T >> 3) + min(l & 7, T & 7) + (l >> 3);
+  // (only where T divides evenly: the persistent kernel's general form cost
+  // the small launches here 0.1 - 0.3 us, and those that it would help by
+  // more have more tiles than CUs and run there)
+  if ((T & 7) == 0) l = (l & 7) * (T >> 3) + (l >> 3);
   // 4 tile-rows per group: the 32 workgroups an XCD runs at once share 4
   // A panels (8 wide groups re-read a large A once per 4 column tiles: the
   // 16384 x 4096 x 16384 split-bf16 wgrad ran 1.80 ms grouped by 8 against
@@ -398,8 +399,12 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
     src = g.B1 + (g.kwrap_b ? 0 : koff) + int64_t(n1) * g.ldb; ld = g.ldb;
     rows_left = min(N - n1, BN); row_base = srow0 - BM - BN;
   }
-  // a wrapping B region addresses contraction bytes koff + t * kSK modulo kwrap_b
-  const uint32_t kwrap = !kMid && srow0 >= BM ? uint32_t(g.kwrap_b) : 0u;
+  // a wrapping B region addresses contraction bytes koff + t * kSK modulo
+  // kwrap_b (the bf16 products of the weight gradients; the test in
+  // every stage of the FP8 products cost 0.1 - 0.4 us: 300 x 2048 x 1024 8.99
+  // -> 8.57 without it)
+  constexpr bool kWrap = AF == kBF16 && !kMid;
+  const uint32_t kwrap = kWrap && srow0 >= BM ? uint32_t(g.kwrap_b) : 0u;
   const uint32_t nrec =
       rows_left > 0 ? uint32_t(int64_t(rows_left - 1) * ld + (kwrap ? int(kwrap) : K)) : 0u;
   const v4i rsrc = make_rsrc(src, nrec);
@@ -1466,6 +1471,8 @@ TCFP_DEV void persist_tiles(const GemmArgs g) {
   // tile `it` of this workgroup -> (m0, n0)
   auto tile_of = [&](int it, int& m0, int& n0) {
     int l = int(blockIdx.x) + it * int(gridDim.x);
+    // (each XCD a run of adjacent tiles, the first T % 8 of them one more:
+    // in plain order 2256 x 12000 x 3008 bf16 ran 166.3 us against 148.4)
     l = (l & 7) * (T >> 3) + min(l & 7, T & 7) + (l >> 3);
     // groups of 4 tile-rows, as in gemm_nt_dma_kernel (A/B on two boxes
     // against 8: 4096^3 95.4 -> 93.9 us, 8192 x 4096 x 1024 fp32 out
