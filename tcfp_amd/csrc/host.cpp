@@ -15,6 +15,7 @@
 // allocated once and lives as long as the process.
 #include <Python.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>
 
@@ -707,6 +708,15 @@ py::tuple block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, cons
 
 PYBIND11_MODULE(_tcfp_host, m) {
   m.doc() = "Native host path of tcfp_amd.kernels";
+  // torch's errors as torch raises them from Python: a caller that handles
+  // torch.OutOfMemoryError (pybind11 alone would make it a RuntimeError)
+  py::register_local_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const c10::Error&) {
+      torch::translate_exception_to_python(p);
+    }
+  });
   m.def("quantize_per_tensor", &quantize_per_tensor);
   m.def("quantize_per_tensor_colsum", &quantize_per_tensor_colsum);
   m.def("dual_quantize_per_tensor", &dual_quantize_per_tensor);

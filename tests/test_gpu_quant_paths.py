@@ -131,3 +131,11 @@ def test_mlp_without_autograd(dev):
     with torch.no_grad():
         out = mlp(x)
     assert torch.equal(out, ref.detach()) and not out.requires_grad
+
+
+def test_out_of_memory_is_torchs_own_error(dev):
+    # 4 TiB once contiguous: the allocator refuses it
+    x = torch.zeros(1, 1, device=dev).expand(2**20, 2**20)
+    with pytest.raises(torch.OutOfMemoryError):
+        K.block_quantize_fp8(x, 64)
+    assert K.block_quantize_fp8(x[:8, :64], 64)[0].shape == (8, 64)
