@@ -2477,7 +2477,9 @@ bool exps_al16(const GemmArgs& ga) {
 // us at 8192 x 4096, 23.2 against 21.9 at 12288; 32 rows 21.5 against 22.2),
 // up to 64 rows, whose activation tile every workgroup reads again, 2048
 // (6.6 against 7.4 us at 2048 x 1024, level at 2048 x 4096; 15.0 against 13.8
-// at 4096 x 4096).
+// at 4096 x 4096).  On codes cold in HBM (a whole serving call, stream against
+// tiles, N 16384): up to 16 rows K 4096 37.5 against 40.2 and block 64 37.0
+// against 37.9, but K 1024 16.2 against 13.1; 32 rows 44.8 against 41.0.
 bool skinny_eligible(const GemmArgs& ga, bool exps) {
   if (g_tile_policy != 0 || ga.M > 64 || ga.N > (ga.M <= 32 ? 8192 : 2048)) return false;
   if (ga.kwrap_b || (ga.kc > 0 && ga.kc < ga.K)) return false;
