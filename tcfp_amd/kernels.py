@@ -306,8 +306,9 @@ def dual_quantize_per_tensor(
     if (stochastic_lo or stochastic_hi) and seed is None:
         seed = int(torch.randint(0, 2**62, (1,)).item())
     if sigma_factor is None:
+        # (any integer seed: its low 64 bits, as the C ABI's other callers pass it)
         return _hip.host().dual_quantize_per_tensor(weight, error_buf, update_ef, stochastic_lo,
-                                                    transposed, seed or 0)
+                                                    transposed, int(seed or 0) & (2**64 - 1))
     dev = _hip.require_gpu(weight, error_buf)
     assert weight.dim() == 2, "weight must be 2-D (N, K)"
     w = weight if weight.is_contiguous() else weight.contiguous()
