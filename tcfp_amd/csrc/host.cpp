@@ -10,9 +10,13 @@
 //
 // The functions keep their Python predecessors' semantics: the same checks in
 // the same order with the same exception types, the same outputs, the
-// current stream of the tensors' device.  Scratch for the reductions is one
-// buffer per (device, stream), as stream order makes its reuse safe; it is
-// allocated once and lives as long as the process.
+// current stream of the tensors' device.  They run without the GIL, which
+// torch.empty and a ctypes call release too: an allocation may wait for the
+// GPU, a launch for room in its queue, and Python's other threads go on.  So
+// nothing in them touches a Python object; results and errors become Python's
+// at the boundary (Outs, Raise).  Scratch for the reductions is one buffer per
+// (device, stream), as stream order makes its reuse safe; it is allocated
+// once and lives as long as the process.
 #include <Python.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -35,14 +39,21 @@ namespace py = pybind11;
 using at::Tensor;
 using OptT = std::optional<Tensor>;
 
-[[noreturn]] void raise(PyObject* type, const std::string& msg) {
-  PyErr_SetString(type, msg.c_str());
-  throw py::error_already_set();
-}
+// A Python exception to be raised at the boundary.
+struct Raise {
+  PyObject* type;
+  std::string msg;
+};
+[[noreturn]] void raise(PyObject* type, const std::string& msg) { throw Raise{type, msg}; }
 [[noreturn]] void assertion(const std::string& m) { raise(PyExc_AssertionError, m); }
 [[noreturn]] void value_error(const std::string& m) { raise(PyExc_ValueError, m); }
 [[noreturn]] void type_error(const std::string& m) { raise(PyExc_TypeError, m); }
 [[noreturn]] void runtime_error(const std::string& m) { raise(PyExc_RuntimeError, m); }
+
+// A tuple of tensors, None where undefined.
+struct Outs {
+  std::vector<Tensor> t;
+};
 
 std::string shape_str(at::IntArrayRef s) {
   std::string r = "(";
@@ -153,22 +164,50 @@ Tensor scalar(const Tensor& t, const char* name) {
 }
 
 // ---- reduction scratch: one per (device, stream) --------------------------
-std::mutex g_ws_mu;
-using WsMap = std::map<std::pair<int, void*>, Tensor>;
+struct Scratch {
+  std::mutex mu;
+  Tensor t;
+};
+std::mutex g_ws_mu;  // of the maps
+using WsMap = std::map<std::pair<int, void*>, Scratch>;
 // (never destroyed: tensors must not outlive the allocator at exit)
 WsMap& ws_map(int kind) {
   static WsMap* const m = new WsMap[2];
   return m[kind];
 }
 
-Tensor workspace(const OnGpu& g, void* stream, bool batch) {
-  std::lock_guard<std::mutex> lk(g_ws_mu);
-  Tensor& t = ws_map(batch ? 1 : 0)[{int(g.device().index()), stream}];
-  if (!t.defined())
-    t = g.empty({int64_t(batch ? tcfp_quantize_batch_workspace_bytes(4) : tcfp_workspace_bytes())},
-                at::kByte);
-  return t;
-}
+// A call's hold on its stream's scratch, to be taken after its allocations and
+// kept over its launches: another thread's call on the same stream enqueues
+// its own before or after all of them.  The scratch is allocated
+// outside the locks, as a dispatch mode's Python code may run there.
+class Workspace {
+ public:
+  Workspace(const OnGpu& g, void* stream, bool batch) {
+    Scratch* s;
+    {
+      std::lock_guard<std::mutex> lk(g_ws_mu);
+      s = &ws_map(batch ? 1 : 0)[{int(g.device().index()), stream}];
+    }
+    lock_ = std::unique_lock<std::mutex>(s->mu);
+    if (!s->t.defined()) {
+      lock_.unlock();
+      Tensor t = g.empty({int64_t(batch ? tcfp_quantize_batch_workspace_bytes(4)
+                                        : tcfp_workspace_bytes())},
+                         at::kByte);
+      lock_.lock();
+      if (!s->t.defined()) s->t = t;
+    }
+    p_ = s->t.data_ptr();
+    n_ = size_t(s->t.numel());
+  }
+  void* ptr() const { return p_; }
+  size_t bytes() const { return n_; }
+
+ private:
+  std::unique_lock<std::mutex> lock_;
+  void* p_;
+  size_t n_;
+};
 
 struct View2d {
   Tensor t;
@@ -184,30 +223,31 @@ View2d as_2d(const Tensor& x) {
 
 // ---- per-tensor quantisation -------------------------------------------------
 
-py::tuple quantize_per_tensor(const Tensor& x, at::ScalarType fp8, const OptT& scale,
+Outs quantize_per_tensor(const Tensor& x, at::ScalarType fp8, const OptT& scale,
                               bool transpose, bool return_scale) {
   OnGpu g;
   g.add(x);
   g.add(scale);
   const View2d v = as_2d(x);
   const int dt = in_dtype(v.t), fmt = fmt_of(fp8);
-  Tensor q = g.empty(x.sizes(), fp8), q_t, s_out, s_in, ws;
+  Tensor q = g.empty(x.sizes(), fp8), q_t, s_out, s_in;
   if (transpose) q_t = g.empty({v.cols, v.rows}, fp8);
   Tensor inv = g.empty({1}, at::kFloat);
   if (return_scale) s_out = g.empty({1}, at::kFloat);
   void* st = g.stream();
+  std::optional<Workspace> ws;
   if (scale) s_in = scalar(scale->to(at::kFloat), "scale");
-  else ws = workspace(g, st, false);
+  else ws.emplace(g, st, false);
   check(tcfp_quantize_per_tensor(ptr(v.t), dt, v.rows, v.cols, fmt, f32(s_in), bytes(q),
-                                 bytes(q_t), f32(s_out), f32(inv), ptr(ws), st),
+                                 bytes(q_t), f32(s_out), f32(inv), ws ? ws->ptr() : nullptr, st),
         "quantize_per_tensor");
-  if (transpose && return_scale) return py::make_tuple(q, inv, q_t, s_out);
-  if (transpose) return py::make_tuple(q, inv, q_t);
-  if (return_scale) return py::make_tuple(q, inv, s_out);
-  return py::make_tuple(q, inv);
+  if (transpose && return_scale) return {{q, inv, q_t, s_out}};
+  if (transpose) return {{q, inv, q_t}};
+  if (return_scale) return {{q, inv, s_out}};
+  return {{q, inv}};
 }
 
-py::tuple quantize_per_tensor_colsum(const Tensor& x, at::ScalarType fp8, bool transpose) {
+Outs quantize_per_tensor_colsum(const Tensor& x, at::ScalarType fp8, bool transpose) {
   OnGpu g({&x});
   const View2d v = as_2d(x);
   if (v.cols % 8 != 0)
@@ -219,12 +259,12 @@ py::tuple quantize_per_tensor_colsum(const Tensor& x, at::ScalarType fp8, bool t
   const size_t n = tcfp_colsum_workspace_bytes(v.rows, v.cols);
   Tensor cws = g.empty({int64_t(std::max<size_t>(n, 16))}, at::kByte);
   void* st = g.stream();
-  Tensor ws = workspace(g, st, false);
+  const Workspace ws(g, st, false);
   check(tcfp_quantize_per_tensor_colsum(ptr(v.t), dt, v.rows, v.cols, fmt, bytes(q), bytes(q_t),
-                                        f32(inv), f32(cs), ptr(ws), ptr(cws), n, st),
+                                        f32(inv), f32(cs), ws.ptr(), ptr(cws), n, st),
         "quantize_per_tensor_colsum");
-  if (transpose) return py::make_tuple(q, inv, q_t, cs);
-  return py::make_tuple(q, inv, cs);
+  if (transpose) return {{q, inv, q_t, cs}};
+  return {{q, inv, cs}};
 }
 
 void check_ef(const Tensor& ef, int64_t n, int64_t k) {
@@ -236,7 +276,7 @@ void check_ef(const Tensor& ef, int64_t n, int64_t k) {
 }
 
 // The amax-rule dual quantisation (no NF-aware scaling).
-py::tuple dual_quantize_per_tensor(const Tensor& weight, const OptT& error_buf, bool update_ef,
+Outs dual_quantize_per_tensor(const Tensor& weight, const OptT& error_buf, bool update_ef,
                                    bool stochastic_lo, bool transposed, uint64_t seed) {
   OnGpu g;
   g.add(weight);
@@ -254,13 +294,13 @@ py::tuple dual_quantize_per_tensor(const Tensor& weight, const OptT& error_buf, 
     lo_t = g.empty({k, n}, e4);
   }
   void* st = g.stream();
-  Tensor ws = workspace(g, st, false);
+  const Workspace ws(g, st, false);
   check(tcfp_dual_quantize_per_tensor(ptr(w), dt, n, k, f32(opt(error_buf)), update_ef ? 1 : 0,
                                       stochastic_lo ? 1 : 0, seed, 0, bytes(hi), bytes(lo),
-                                      f32(ih), f32(il), bytes(hi_t), bytes(lo_t), ptr(ws), st),
+                                      f32(ih), f32(il), bytes(hi_t), bytes(lo_t), ws.ptr(), st),
         "dual_quantize_per_tensor");
-  if (transposed) return py::make_tuple(hi, lo, ih, il, hi_t, lo_t);
-  return py::make_tuple(hi, lo, ih, il);
+  if (transposed) return {{hi, lo, ih, il, hi_t, lo_t}};
+  return {{hi, lo, ih, il}};
 }
 
 // (weight, error_buf, update_ef, transposed) and (x, fp8_dtype, transpose)
@@ -268,7 +308,7 @@ using DualIn = std::tuple<Tensor, OptT, bool, bool>;
 using ActIn = std::tuple<Tensor, at::ScalarType, bool>;
 
 // The batch itself (its caller has checked that every tensor fits).
-std::pair<py::list, py::list> quantize_batch(const std::vector<DualIn>& dual,
+std::pair<std::vector<Outs>, std::vector<Outs>> quantize_batch(const std::vector<DualIn>& dual,
                                              const std::vector<ActIn>& act) {
   if (dual.size() + act.size() > 4) value_error("at most four tensors in a batch");
   OnGpu g;
@@ -281,7 +321,7 @@ std::pair<py::list, py::list> quantize_batch(const std::vector<DualIn>& dual,
   tcfp_quant_job jobs[4] = {};
   std::vector<Tensor> held;  // contiguous copies, alive until the launch
   int nj = 0;
-  py::list rd, ra;
+  std::vector<Outs> rd, ra;
   const at::ScalarType e4 = at::kFloat8_e4m3fn;
   for (const auto& d : dual) {
     Tensor w = std::get<0>(d);
@@ -311,8 +351,8 @@ std::pair<py::list, py::list> quantize_batch(const std::vector<DualIn>& dual,
     j.q_lo = bytes(lo);
     j.q_lo_t = bytes(lt);
     j.inv_lo = f32(il);
-    if (t) rd.append(py::make_tuple(hi, lo, ih, il, ht, lt));
-    else rd.append(py::make_tuple(hi, lo, ih, il));
+    if (t) rd.push_back({{hi, lo, ih, il, ht, lt}});
+    else rd.push_back({{hi, lo, ih, il}});
   }
   for (const auto& a : act) {
     Tensor x = std::get<0>(a);
@@ -334,12 +374,12 @@ std::pair<py::list, py::list> quantize_batch(const std::vector<DualIn>& dual,
     j.q = bytes(q);
     j.q_t = bytes(qt);
     j.inv = f32(inv);
-    if (std::get<2>(a)) ra.append(py::make_tuple(q, inv, qt));
-    else ra.append(py::make_tuple(q, inv));
+    if (std::get<2>(a)) ra.push_back({{q, inv, qt}});
+    else ra.push_back({{q, inv}});
   }
   void* st = g.stream();
-  Tensor ws = workspace(g, st, true);
-  check(tcfp_quantize_batch(nj, jobs, ptr(ws), size_t(ws.numel()), st), "quantize_batch");
+  const Workspace ws(g, st, true);
+  check(tcfp_quantize_batch(nj, jobs, ws.ptr(), ws.bytes(), st), "quantize_batch");
   return {rd, ra};
 }
 
@@ -386,7 +426,7 @@ Tensor dual_gemm(const Tensor& a_, const Tensor& b_hi_, const OptT& b_lo_, const
   return out;
 }
 
-py::tuple block_quantize(const Tensor& x_, int64_t bs, at::ScalarType fp8, bool f32s) {
+Outs block_quantize(const Tensor& x_, int64_t bs, at::ScalarType fp8, bool f32s) {
   OnGpu g({&x_});
   if (x_.dim() != 2) value_error("expected a 2-D tensor");
   const int64_t m = x_.size(0), k = x_.size(1);
@@ -404,7 +444,7 @@ py::tuple block_quantize(const Tensor& x_, int64_t bs, at::ScalarType fp8, bool 
                       : tcfp_block_quantize(ptr(x), dt, m, k, int(bs), fmt, bytes(q), exps(s),
                                             g.stream());
   check(rc, "block_quantize_fp8");
-  return py::make_tuple(q, s);
+  return {{q, s}};
 }
 
 Tensor block_scales(const Tensor& e, int64_t rows, int64_t nkb, const char* name,
@@ -487,7 +527,7 @@ GemmOps gemm_operands(const Tensor& a_, const Tensor& b_hi_, const Tensor& b_lo_
   return o;
 }
 
-py::tuple dual_gemm_gelu_quantize(const Tensor& a_, const Tensor& b_hi_, const Tensor& b_lo_,
+Outs dual_gemm_gelu_quantize(const Tensor& a_, const Tensor& b_hi_, const Tensor& b_lo_,
                                   const Tensor& s_a, const Tensor& s_hi, const Tensor& s_lo,
                                   const OptT& bias, at::ScalarType fp8, bool transpose,
                                   bool return_act, bool return_dgelu) {
@@ -510,23 +550,20 @@ py::tuple dual_gemm_gelu_quantize(const Tensor& a_, const Tensor& b_hi_, const T
   const Tensor sa = scalar(s_a, "scale_a"), sh = scalar(s_hi, "scale_hi"),
                sl = scalar(s_lo, "scale_lo");
   void* st = g.stream();
-  Tensor ws = workspace(g, st, false);
+  const Workspace ws(g, st, false);
   check(tcfp_dual_gemm_gelu_quantize(
             bytes(o.a), fmt_of(o.a.scalar_type()), o.a.stride(0), bytes(o.b_hi), bytes(o.b_lo),
             fmt_of(o.b_hi.scalar_type()), o.b_hi.stride(0), m, n, k, f32(sa), f32(sh), f32(sl),
-            f32(b), f32(h), f32(act), f32(dg), fmt, bytes(q), bytes(q_t), f32(inv), ptr(ws), st),
+            f32(b), f32(h), f32(act), f32(dg), fmt, bytes(q), bytes(q_t), f32(inv), ws.ptr(), st),
         "dual_gemm_gelu_quantize");
-  py::list r;
-  r.append(h);
-  r.append(q);
-  r.append(inv);
-  if (transpose) r.append(q_t);
-  if (return_act) r.append(act);
-  if (return_dgelu) r.append(dg);
-  return py::tuple(r);
+  Outs r{{h, q, inv}};
+  if (transpose) r.t.push_back(q_t);
+  if (return_act) r.t.push_back(act);
+  if (return_dgelu) r.t.push_back(dg);
+  return r;
 }
 
-py::tuple dual_gemm_dgelu_quantize_colsum(const Tensor& a_, const Tensor& b_hi_,
+Outs dual_gemm_dgelu_quantize_colsum(const Tensor& a_, const Tensor& b_hi_,
                                           const Tensor& b_lo_, const Tensor& s_a,
                                           const Tensor& s_hi, const Tensor& s_lo,
                                           const Tensor& dgelu, at::ScalarType fp8, bool transpose,
@@ -556,25 +593,23 @@ py::tuple dual_gemm_dgelu_quantize_colsum(const Tensor& a_, const Tensor& b_hi_,
   const Tensor sa = scalar(s_a, "scale_a"), sh = scalar(s_hi, "scale_hi"),
                sl = scalar(s_lo, "scale_lo");
   void* st = g.stream();
-  Tensor ws = workspace(g, st, false);
+  const Workspace ws(g, st, false);
   check(tcfp_dual_gemm_dgelu_quantize_colsum(
             bytes(o.a), fmt_of(o.a.scalar_type()), o.a.stride(0), bytes(o.b_hi), bytes(o.b_lo),
             fmt_of(o.b_hi.scalar_type()), o.b_hi.stride(0), m, n, k, f32(sa), f32(sh), f32(sl),
-            f32(dc), f32(gr), fmt, bytes(q), bytes(q_t), f32(inv), f32(cs), ptr(ws), ptr(cws),
+            f32(dc), f32(gr), fmt, bytes(q), bytes(q_t), f32(inv), f32(cs), ws.ptr(), ptr(cws),
             nbytes, st),
         "dual_gemm_dgelu_quantize_colsum");
-  py::list r;
-  r.append(codes ? py::cast(q) : py::object(py::none()));
-  r.append(inv);
-  if (transpose) r.append(q_t);
-  if (col_sum) r.append(cs);
-  if (return_grad) r.append(gr);
-  return py::tuple(r);
+  Outs r{{q, inv}};
+  if (transpose) r.t.push_back(q_t);
+  if (col_sum) r.t.push_back(cs);
+  if (return_grad) r.t.push_back(gr);
+  return r;
 }
 
 // ---- the block-scaled layer -------------------------------------------------------
 
-py::tuple block_linear_forward(const Tensor& x2d, const Tensor& weight, const OptT& bias,
+Outs block_linear_forward(const Tensor& x2d, const Tensor& weight, const OptT& bias,
                                int64_t bs, const OptT& error_buf, bool srr, bool update_ef,
                                uint64_t seed) {
   if (bs != 32 && bs != 64 && bs != 128)
@@ -618,7 +653,7 @@ py::tuple block_linear_forward(const Tensor& x2d, const Tensor& weight, const Op
                                ptr(out), TCFP_DTYPE_F32, N, st),
           "block_dual_gemm");
   }
-  return py::make_tuple(out, hi, lo, eh, el, aq, ae);
+  return {{out, hi, lo, eh, el, aq, ae}};
 }
 
 // G^T deq(X) to fp32 accuracy for any token count: per-tensor codes with their
@@ -649,7 +684,7 @@ Tensor wgrad_f32(const Tensor& grad, const Tensor& act, const OptT& inv, const O
   return dw;
 }
 
-py::tuple block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, const OptT& act_e,
+Outs block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, const OptT& act_e,
                                 const OptT& w_hi, const OptT& w_lo, const OptT& e_hi,
                                 const OptT& e_lo, int64_t bs, bool need_dx, bool need_dw,
                                 bool want_db, bool split_lo, at::ScalarType dx_dtype) {
@@ -698,35 +733,53 @@ py::tuple block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, cons
                                           out_dtype_of(dx_dtype), ptr(ws), n, st),
           "block_dgrad_from_prep");
   }
-  auto ret = [](const Tensor& t) -> py::object {
-    return t.defined() ? py::cast(t) : py::object(py::none());
-  };
-  return py::make_tuple(ret(dx), ret(dw), ret(db));
+  return {{dx, dw, db}};
 }
 
 }  // namespace
 
+namespace pybind11::detail {
+template <>
+struct type_caster<Outs> {
+  PYBIND11_TYPE_CASTER(Outs, const_name("tuple"));
+  bool load(handle, bool) { return false; }  // results only
+  static handle cast(const Outs& o, return_value_policy, handle) {
+    tuple r(o.t.size());
+    for (size_t i = 0; i < o.t.size(); ++i)
+      r[i] = o.t[i].defined() ? pybind11::cast(o.t[i]) : object(none());
+    return r.release();
+  }
+};
+}  // namespace pybind11::detail
+
 PYBIND11_MODULE(_tcfp_host, m) {
   m.doc() = "Native host path of tcfp_amd.kernels";
   // torch's errors as torch raises them from Python: a caller that handles
-  // torch.OutOfMemoryError (pybind11 alone would make it a RuntimeError)
+  // torch.OutOfMemoryError, or the exception that its dispatch mode raised
+  // (pybind11 alone would make each a RuntimeError)
   py::register_local_exception_translator([](std::exception_ptr p) {
     try {
       if (p) std::rethrow_exception(p);
+    } catch (const Raise& e) {
+      PyErr_SetString(e.type, e.msg.c_str());
+    } catch (python_error& e) {
+      e.restore();
     } catch (const c10::Error&) {
       torch::translate_exception_to_python(p);
     }
   });
-  m.def("quantize_per_tensor", &quantize_per_tensor);
-  m.def("quantize_per_tensor_colsum", &quantize_per_tensor_colsum);
-  m.def("dual_quantize_per_tensor", &dual_quantize_per_tensor);
-  m.def("quantize_batch", &quantize_batch);
-  m.def("dual_gemm", &dual_gemm);
-  m.def("block_quantize", &block_quantize);
-  m.def("block_gemm", &block_gemm);
-  m.def("dual_gemm_gelu_quantize", &dual_gemm_gelu_quantize);
-  m.def("dual_gemm_dgelu_quantize_colsum", &dual_gemm_dgelu_quantize_colsum);
-  m.def("wgrad_f32", &wgrad_f32);
-  m.def("block_linear_forward", &block_linear_forward);
-  m.def("block_linear_backward", &block_linear_backward);
+  // (results are converted after the guard has taken the GIL back)
+  using NoGil = py::call_guard<py::gil_scoped_release>;
+  m.def("quantize_per_tensor", &quantize_per_tensor, NoGil());
+  m.def("quantize_per_tensor_colsum", &quantize_per_tensor_colsum, NoGil());
+  m.def("dual_quantize_per_tensor", &dual_quantize_per_tensor, NoGil());
+  m.def("quantize_batch", &quantize_batch, NoGil());
+  m.def("dual_gemm", &dual_gemm, NoGil());
+  m.def("block_quantize", &block_quantize, NoGil());
+  m.def("block_gemm", &block_gemm, NoGil());
+  m.def("dual_gemm_gelu_quantize", &dual_gemm_gelu_quantize, NoGil());
+  m.def("dual_gemm_dgelu_quantize_colsum", &dual_gemm_dgelu_quantize_colsum, NoGil());
+  m.def("wgrad_f32", &wgrad_f32, NoGil());
+  m.def("block_linear_forward", &block_linear_forward, NoGil());
+  m.def("block_linear_backward", &block_linear_backward, NoGil());
 }
