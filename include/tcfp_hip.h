@@ -577,7 +577,8 @@ int tcfp_block_wgrad(const float* g, int64_t m, int64_t n_out, const uint8_t* x,
  * per-tensor inverse scale `inv` (device scalar; NULL: 1) or block exponents
  * e_x [k_in / block, m] (NULL: none).  The fp32 matmuls that the reference
  * runs where its FP8 product does not apply (tcfp/nn/__init__.py:553-555,
- * 743-750), as three exact bf16 passes.  dw [n_out, k_in] fp32.  Workspace:
+ * 743-750), as three exact bf16 passes; the scale's power of two multiplies
+ * the codes ahead of the sum, so only results past fp32's range overflow.  dw [n_out, k_in] fp32.  Workspace:
  * tcfp_wgrad_f32_workspace_bytes(m, n_out, k_in). */
 size_t tcfp_wgrad_f32_workspace_bytes(int64_t m, int64_t n_out, int64_t k_in);
 int tcfp_wgrad_f32(const float* g, int64_t m, int64_t n_out, const uint8_t* x, int x_fmt,

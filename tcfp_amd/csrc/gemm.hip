@@ -3540,7 +3540,11 @@ int wgrad_chunked(const uint16_t* ap, int64_t m, int64_t n_out, const uint8_t* x
 // product is three bf16 passes over one copy of X with fp32 accumulation,
 //   A' = [g1 | g2 | g3]^T  [n_out, 3 mp],   B' = x^T  [k_in, mp],
 // mp = m rounded up to 64 (zeros behind), where an fp32 matrix product runs
-// at a sixteenth of the bf16 rate.  A per-tensor scale goes into the epilogue.
+// at a sixteenth of the bf16 rate.  Of a per-tensor scale the power of two goes
+// into the codes, exactly, and the rest (1 to 2) into the epilogue: the sums
+// stay below the result, so what the fp32 form holds does not overflow here.
+// (An inf code of X next to a zero part gives NaN where the fp32 form gives inf:
+// no quantiser here writes one.)
 // (With the dequantising copies of the fp32 form: 1000 tokens, 1040 -> 1552,
 // 53 -> 40 us; 2000 tokens, 4096 -> 8192, 936 -> 473; 1999 tokens, 1024 -> 4096,
 // 138 -> 75; 201 tokens, 256 -> 512, 31 -> 18.5.  Errors against 64 bits 1e-7
@@ -3611,15 +3615,26 @@ __global__ __launch_bounds__(256) void split3_t_bf16_kernel(const float* __restr
   }
 }
 
-// out[c, r] = bf16(q[r, c] * 2^e[c / bs, r]) (e null: the codes' values), r <
-// mp, rows past m zero.
+// out[c, r] = bf16(q[r, c] * 2^e[c / bs, r]), r < mp, rows past m zero; with
+// e null bf16(q[r, c] * 2^p), p the exponent of *inv (inv null: 0), held to
+// where a code times 2^p is a normal bf16, and *rest = *inv / 2^p.
 template <int FMT>
 __global__ __launch_bounds__(256) void codes_t_bf16_kernel(const uint8_t* __restrict__ q,
                                                            const int8_t* __restrict__ e,
+                                                           const float* __restrict__ inv,
                                                            int64_t m, int64_t k, int bs_shift,
                                                            int64_t mp, bool vec,
-                                                           uint16_t* __restrict__ out) {
+                                                           uint16_t* __restrict__ out,
+                                                           float* __restrict__ rest) {
   __shared__ uint16_t tile[64][64 + 2];
+  float pw = 1.0f;
+  if (inv) {
+    const float s = *inv;
+    const int ex = int((__float_as_uint(s) >> 23) & 0xFFu);
+    const int p = e || ex == 0xFF ? 0 : min(max(ex - 127, -100), 100);
+    pw = exp2i(p);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *rest = s * exp2i(-p);
+  }
   const int tiles_c = int((k + 63) / 64);
   const int64_t r0 = int64_t(blockIdx.x / tiles_c) * 64, c0 = int64_t(blockIdx.x % tiles_c) * 64;
   const int t = threadIdx.x;
@@ -3628,7 +3643,7 @@ __global__ __launch_bounds__(256) void codes_t_bf16_kernel(const uint8_t* __rest
     const int64_t r = r0 + lr;
     if (vec && r < m && c0 + lc + 16 <= k) {
       const uint4 w = *reinterpret_cast<const uint4*>(q + r * k + c0 + lc);
-      deq16_to_tile<FMT>(w, e ? exp2i(e[((c0 + lc) >> bs_shift) * m + r]) : 1.0f, tile, lc, lr);
+      deq16_to_tile<FMT>(w, e ? exp2i(e[((c0 + lc) >> bs_shift) * m + r]) : pw, tile, lc, lr);
     } else {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
@@ -3636,7 +3651,7 @@ __global__ __launch_bounds__(256) void codes_t_bf16_kernel(const uint8_t* __rest
         uint16_t v = 0;
         if (r < m && c < k)
           v = f32_to_bf16_rne(fp8_to_f32<FMT>(q[r * k + c]) *
-                              (e ? exp2i(e[(c >> bs_shift) * m + r]) : 1.0f));
+                              (e ? exp2i(e[(c >> bs_shift) * m + r]) : pw));
         tile[lc + j][lr] = v;
       }
     }
@@ -3665,7 +3680,8 @@ size_t f32w_part_bytes(int64_t m, int64_t rows, int64_t k_in) {
 size_t f32w_ws_bytes(int64_t m, int64_t n_out, int64_t k_in) {
   const int64_t mp = f32w_mp(m), rows = f32w_rows(m, n_out);
   const int64_t rem = rows > 0 ? n_out % rows : 0;
-  return align256(size_t(k_in) * size_t(mp) * 2) + align256(size_t(rows) * size_t(mp) * 6) +
+  // (256: the scale's rest)
+  return 256 + align256(size_t(k_in) * size_t(mp) * 2) + align256(size_t(rows) * size_t(mp) * 6) +
          std::max(f32w_part_bytes(m, rows, k_in), rem ? f32w_part_bytes(m, rem, k_in) : 0);
 }
 
@@ -3994,6 +4010,8 @@ extern "C" int tcfp_wgrad_f32(const float* g, int64_t m, int64_t n_out, const ui
   const int64_t mp = f32w_mp(m), rows = f32w_rows(m, n_out);
   const int shift = block == 32 ? 5 : (block == 64 ? 6 : 7);
   uint8_t* ws = static_cast<uint8_t*>(workspace);
+  float* rest = reinterpret_cast<float*>(ws);
+  ws += 256;
   uint16_t* xt = reinterpret_cast<uint16_t*>(ws);
   ws += align256(size_t(k_in) * size_t(mp) * 2);
   uint16_t* gs = reinterpret_cast<uint16_t*>(ws);
@@ -4002,9 +4020,11 @@ extern "C" int tcfp_wgrad_f32(const float* g, int64_t m, int64_t n_out, const ui
   if (!grid_x_fits(tx, 256)) return TCFP_ERR_SHAPE;
   const bool vec = al16(x);
   if (x_fmt == TCFP_FP8_E5M2)
-    codes_t_bf16_kernel<TCFP_FP8_E5M2><<<unsigned(tx), 256, 0, st>>>(x, e_x, m, k_in, shift, mp, vec, xt);
+    codes_t_bf16_kernel<TCFP_FP8_E5M2><<<unsigned(tx), 256, 0, st>>>(x, e_x, inv, m, k_in, shift,
+                                                                    mp, vec, xt, rest);
   else
-    codes_t_bf16_kernel<TCFP_FP8_E4M3><<<unsigned(tx), 256, 0, st>>>(x, e_x, m, k_in, shift, mp, vec, xt);
+    codes_t_bf16_kernel<TCFP_FP8_E4M3><<<unsigned(tx), 256, 0, st>>>(x, e_x, inv, m, k_in, shift,
+                                                                    mp, vec, xt, rest);
   for (int64_t c0 = 0; c0 < n_out; c0 += rows) {
     const int64_t n = std::min(rows, n_out - c0);
     const int64_t tg = (mp / 64) * ((n + 63) / 64);
@@ -4016,7 +4036,7 @@ extern "C" int tcfp_wgrad_f32(const float* g, int64_t m, int64_t n_out, const ui
     ga.B0 = ga.B1 = reinterpret_cast<const uint8_t*>(xt);
     ga.M = int(n); ga.N = int(k_in); ga.K = int(6 * mp);
     ga.lda = 6 * mp; ga.ldb = 2 * mp; ga.kwrap_b = int(2 * mp);
-    ga.s_a = inv;
+    ga.s_a = inv ? rest : nullptr;
     ga.out = dw + c0 * k_in; ga.ldo = k_in;
     int64_t kc;
     const int64_t splits = wgrad_splits_of(6 * mp, n, k_in, &kc);

@@ -54,6 +54,12 @@ def test_block(dev, m, bs):
     assert _rel(dw, ref) <= max(1.2 * _rel(g.t() @ xd, ref), 2e-7)
 
 
+def _same(x, ref):
+    """Equal values, NaN equal to NaN, an inf only to the same inf."""
+    return torch.equal(x.isnan(), ref.isnan()) and torch.equal(
+        torch.where(x.isnan(), 0, x), torch.where(ref.isnan(), 0, ref))
+
+
 def test_special_gradients(dev):
     """Non-finite and extreme gradients as the fp32 product has them: an inf
     row stays inf, a NaN NaN, the largest and smallest normals are exact."""
@@ -66,10 +72,30 @@ def test_special_gradients(dev):
     g[5, 2] = torch.finfo(torch.float32).max
     g[6, 3] = -1.2345678e-20
     g[7, 4] = float("-inf")
+    g[8, 5] = torch.finfo(torch.float32).tiny
     dw = K.wgrad_f32(g, q, inv)
-    ref = g.t() @ q.float()
-    assert torch.equal(dw.isnan(), ref.isnan())
-    assert torch.equal(dw.nan_to_num(), ref.nan_to_num())
+    assert _same(dw, g.t() @ q.float())
+
+
+@pytest.mark.parametrize("inv", [0.0123, 2.0**-60, 1.7e-38, 3.0, 5e8, float("nan")])
+@pytest.mark.parametrize("fp8", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_scale_ahead_of_the_sum(dev, inv, fp8):
+    """Gradients whose products with the codes pass fp32's range where those
+    with the scaled codes do not, and the reverse: finite where the fp32
+    product is, to the same accuracy."""
+    m, n, k = 35, 48, 64
+    gen = torch.Generator().manual_seed(7)
+    q = (torch.randn(m, k, generator=gen) * 100).to(fp8).to(dev)
+    s = torch.full((1,), inv, device=dev)
+    # (products up to 2e36 * 4 * 400 > 3.4e38; results of 35 terms of deviation 2e36 *
+    # 100 * 0.0123 stay ten deviations, 1.5e37 each, inside the range, whatever the order)
+    mag = 2e36 if inv < 1 else 1e30 / inv
+    g = (torch.randn(m, n, generator=gen) * mag).to(dev)
+    dw, ref = K.wgrad_f32(g, q, s), g.double().t() @ (q.double() * s.double())
+    fp32 = g.t() @ (q.float() * s)
+    assert torch.equal(dw.isfinite(), fp32.isfinite())
+    if fp32.isfinite().any():
+        assert _rel(dw, ref) <= max(1.2 * _rel(fp32, ref), 2e-7)
 
 
 def test_layer_uses_it(dev):
