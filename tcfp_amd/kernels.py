@@ -1124,6 +1124,16 @@ def fused_block_scaled_dual_gemm_backward_dx(
                                           w_lo_scales, block_size)
 
 
+def _in_transform(grad: torch.Tensor) -> bool:
+    """Whether a graph is being recorded over ``grad`` (a backward under
+    ``create_graph``) or it is a batch (``is_grads_batched``, a backward under
+    ``vmap``): the odd token counts' weight gradient is torch's fp32 product
+    then, which goes through both."""
+    ft = torch._C._functorch
+    return ((torch.is_grad_enabled() and grad.requires_grad)
+            or ft.is_legacy_batchedtensor(grad) or ft.is_functorch_wrapped_tensor(grad))
+
+
 def block_scaled_wgrad(
     grad: torch.Tensor,
     act_fp8: torch.Tensor,
@@ -1145,6 +1155,8 @@ def block_scaled_wgrad(
     assert M == M2, f"token mismatch: grad {tuple(grad.shape)} vs act {tuple(act_fp8.shape)}"
     dev = _hip.require_gpu(grad, act_fp8, act_scales)
     if M % 4 != 0:
+        if _in_transform(grad):
+            return grad.float().t() @ block_dequantize_fp8(act_fp8, act_scales, block_size)
         return _hip.host().wgrad_f32(grad, act_fp8, None, act_scales, block_size)
     g = grad.float().contiguous()
     a = act_fp8.contiguous()
@@ -1171,7 +1183,10 @@ def wgrad_f32(grad: torch.Tensor, act_fp8: torch.Tensor, act_inv: torch.Tensor) 
     grad [M, N], M >= 1, any count; act [M, K] FP8, K % 16 == 0; act_inv (1,)
     fp32.  The fp32 gradient is the exact sum of three bf16 parts and the codes
     are exact in bf16: three passes on the bf16 MFMA with fp32 accumulation.
+    Differentiable in ``grad``, and batchable over it, as the fp32 matmul is.
     """
+    if _in_transform(grad):
+        return grad.float().t() @ (act_fp8.float() * act_inv)
     return _hip.host().wgrad_f32(grad, act_fp8, act_inv, None, 0)
 
 

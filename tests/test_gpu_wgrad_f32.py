@@ -108,3 +108,40 @@ def test_layer_uses_it(dev):
     q, inv = K.quantize_per_tensor(x)
     ref = g.double().t() @ (q.double() * inv.double())
     assert _rel(layer.weight.grad, ref) < 1e-6
+
+
+@pytest.mark.parametrize("bs", [None, 32])
+def test_layer_under_create_graph(dev, bs):
+    """A gradient penalty on dW at an odd token count: the weight gradient of a
+    frozen input is linear in the output's gradient and can be differentiated.
+    With A the dequantised activation, out's gradient 2 out and s = sum dW^2:
+    ds/dout = 4 A dW^T, and ds/dW = (4 A dW^T)^T A."""
+    torch.manual_seed(0)
+    m = 35
+    layer = TCFPLinear(64, 96, use_tensor_cores=True, scale_block_size=bs, bias=False,
+                       error_feedback=False).to(dev)
+    x = torch.randn(m, 64, device=dev)
+    out = layer(x)
+    dw, = torch.autograd.grad(out.square().sum(), layer.weight, create_graph=True)
+    got, = torch.autograd.grad(dw.square().sum(), layer.weight)
+    a = (K.block_dequantize_fp8(*K.block_quantize_fp8(x, bs), bs) if bs else
+         K.quantize_per_tensor(x)[0].float() * K.quantize_per_tensor(x)[1]).double()
+    ref = (2 * out.detach().double()).t() @ a
+    assert _rel(dw, ref) < 1e-6
+    assert _rel(got, (4 * a @ ref.t()).t() @ a) < 1e-6
+
+
+@pytest.mark.parametrize("bs", [None, 32])
+def test_layer_with_batched_gradients(dev, bs):
+    torch.manual_seed(0)
+    m = 35
+    layer = TCFPLinear(64, 96, use_tensor_cores=True, scale_block_size=bs, bias=False,
+                       error_feedback=False).to(dev)
+    out = layer(torch.randn(m, 64, device=dev))
+    gs = torch.randn(3, m, 96, device=dev)
+    batched, = torch.autograd.grad(out, layer.weight, gs, retain_graph=True, is_grads_batched=True)
+    each = [torch.autograd.grad(out, layer.weight, g, retain_graph=True)[0] for g in gs]
+    mapped = torch.func.vmap(
+        lambda g: torch.autograd.grad(out, layer.weight, g, retain_graph=True)[0])(gs)
+    for b in (batched, mapped):
+        assert _rel(b, torch.stack(each).double()) < 1e-6
