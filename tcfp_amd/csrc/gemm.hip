@@ -2473,15 +2473,23 @@ bool exps_al16(const GemmArgs& ga) {
 
 // The weight stream: few activation rows, whole contraction, descriptors and
 // 32-bit exponent offsets within reach.  Its limit on N is where the 64-column
-// tiles keep enough CUs busy: up to 32 rows 8192 (16 rows: 17.3 against 21.8
-// us at 8192 x 4096, 23.2 against 21.9 at 12288; 32 rows 21.5 against 22.2),
-// up to 64 rows, whose activation tile every workgroup reads again, 2048
-// (6.6 against 7.4 us at 2048 x 1024, level at 2048 x 4096; 15.0 against 13.8
-// at 4096 x 4096).  On codes cold in HBM (a whole serving call, stream against
-// tiles, N 16384): up to 16 rows K 4096 37.5 against 40.2 and block 64 37.0
-// against 37.9, but K 1024 16.2 against 13.1; 32 rows 44.8 against 41.0.
+// tiles keep enough CUs busy.  Each line below, tiles against stream, us, codes
+// cold in HBM and (in brackets) in the caches:
+// * up to 16 rows, N <= 8192: 8192 x 4096 20.3 against 16.6 (13.1, 13.2), x 1024
+//   8.2 against 7.9 (6.4, 6.7); N 16384 x 1024 13.1 against 16.2 cold;
+// * up to 32 rows, N <= 4096, a workgroup per CU: 32 x 4096 x 4096 18.0 against
+//   12.4 (12.5, 9.6).  Above, up to 8192, with short contractions only: per
+//   tensor 32 x 8192 x 512 6.4 against 5.7, but x 2048 11.9 against 11.5 (8.6,
+//   9.7) and x 4096 20.8 against 20.6 (13.4, 17.4; 17 rows 13.1, 15.0); block 64
+//   x 2048 13.0 against 12.4 (11.4, 11.3), but x 4096 22.2 against 22.1 (18.5,
+//   19.4);
+// * up to 64 rows, whose activation tile every workgroup reads again, N <= 2048:
+//   2048 x 4096 18.6 against 14.7 (12.6, 13.1), x 2048 11.6 against 8.7 (8.4,
+//   7.7); 4096 x 4096 (13.8, 15.0).
 bool skinny_eligible(const GemmArgs& ga, bool exps) {
-  if (g_tile_policy != 0 || ga.M > 64 || ga.N > (ga.M <= 32 ? 8192 : 2048)) return false;
+  const bool short_k = ga.K <= (exps ? 2048 : 512);
+  const int max_n = ga.M <= 16 || (ga.M <= 32 && short_k) ? 8192 : (ga.M <= 32 ? 4096 : 2048);
+  if (g_tile_policy != 0 || ga.M > 64 || ga.N > max_n) return false;
   if (ga.kwrap_b || (ga.kc > 0 && ga.kc < ga.K)) return false;
   if (int64_t(64) * ga.lda + ga.K >= kMaxSpan || int64_t(kSkN) * ga.ldb + ga.K >= kMaxSpan)
     return false;

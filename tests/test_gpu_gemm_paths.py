@@ -96,6 +96,33 @@ def test_few_rows_block_exponents(dev, m, n, kb, bs, dual):
         assert err < tol
 
 
+# both sides of the weight stream's lines: 17 to 32 rows and more output columns
+# than CUs x 16, where it pays for short contractions only
+@pytest.mark.parametrize("m,n,k,bs,stream", [
+    (17, 4096, 1040, 0, True), (32, 4112, 512, 0, True), (17, 4112, 528, 0, False),
+    (32, 8192, 4096, 0, False), (17, 4112, 2048, 64, True), (32, 8192, 2176, 128, False)])
+def test_few_rows_of_wide_weights(dev, m, n, k, bs, stream):
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k, generator=g).to(dev), torch.randn(n, k, generator=g).to(dev)
+    if bs:
+        a, ea = K.block_quantize_fp8(x, bs)
+        hi, lo, eh, el = K.fused_dual_quantize_fp8(w, bs)
+        ref = _deq(a, ea, bs) @ (_deq(hi, eh, bs) + _deq(lo, el, bs)).t()
+
+        def run():
+            return K.fused_block_scaled_dual_gemm_forward(a, hi, lo, ea, eh, el, bs)
+    else:
+        a, sa = K.quantize_per_tensor(x)
+        hi, lo, ih, il = K.dual_quantize_per_tensor(w)
+        ref = (a.double() * sa.double()) @ (hi.double() * ih.double()
+                                            + lo.double() * il.double()).t()
+
+        def run():
+            return K.fused_dual_gemm_forward(a, hi, lo, sa, ih, il)
+    assert any("gemm_skinny" in x for x in _kernel_names(run)) == stream
+    assert _rel(run(), ref) < 1e-4
+
+
 @pytest.mark.parametrize("bs", [32, 64, 128])
 @pytest.mark.parametrize("m,n,k", [(100, 130, 640), (257, 500, 768), (1000, 512, 4096),
                                    (65, 96, 1920)])
