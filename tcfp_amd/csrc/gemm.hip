@@ -2523,9 +2523,15 @@ int launch_skinny(const GemmArgs& ga, hipStream_t st) {
 // 6.4 us at 1000 x 4096); launch, first loads and output are ~7 us beside it.
 // Where the line lies: shorter contractions in more than one round lose the
 // overlap of two workgroups' epilogues (per tensor 1100 x 4096 x 4096 55.6 ->
-// 52.0, x 1024 19.2 -> 21.0; 1300 x 4096 x 2048 29.8 -> 30.3; one round, K 1024,
-// 13.5 -> 13.2, K 512 10.7 -> 10.9; block 64 2048 x 2048 x 512 12.2 -> 10.7, x 256
-// level, 1500 x 4096 x 512 18.4 -> 18.9, 520 x 8192 x 1024 27.1 -> 23.0).
+// 52.0, x 1024 19.2 -> 21.0; 1300 x 4096 x 2048 29.8 -> 30.3).  In one round,
+// per tensor, as part of a serving pass (cast and product; codes in the caches,
+// and cold): 1000 x 4096 x 1024 19.0 -> 19.9 and 22.3 -> 22.3, x 1408 21.8 ->
+// 23.7 and 26.3 -> 25.6, x 1536 22.6 -> 23.0 and 28.8 -> 26.8, x 2048 25.2 ->
+// 25.2 and 30.4 -> 28.5, x 4096 41.3 -> 38.3 and 47.7 -> 42.4; rows that do not
+// start on 128-byte lines, which the small tile fetches once more for every 64
+// columns, pay from 1024 on (x 1040 22.0 -> 22.0 and 27.8 -> 26.6, x 1104 24.6 ->
+// 23.3 and 29.1 -> 27.5).  Block 64: 2048 x 2048 x 512 12.2 -> 10.7, x 256
+// level, 1500 x 4096 x 512 18.4 -> 18.9, 520 x 8192 x 1024 27.1 -> 23.0.
 // From one large tile per CU on the large tile is faster (2048 x 4096 x 2048
 // 33.9 against 36.9), and so is the small tile's one round (512 x 4096 x 4096
 // 23.5 against 30.6).  Single products and bf16 operands measured level: not
@@ -2543,7 +2549,9 @@ bool mid_eligible(const GemmArgs& ga, bool exps) {
   const int64_t cus = num_cus();
   if (tiles(256, 128) >= cus || tiles(128, 64) <= cus) return false;
   const bool one_round = tiles(128, 128) <= cus;
-  return exps ? ga.K >= (one_round ? 512 : 1024) : ga.K >= (one_round ? 1024 : 3072);
+  if (exps) return ga.K >= (one_round ? 512 : 1024);
+  const bool lines = ga.lda % 128 == 0 && ga.ldb % 128 == 0;
+  return ga.K >= (one_round ? (lines ? 1536 : 1024) : 3072);
 }
 
 template <int AF, int BF, typename OutT, int SCALE>

@@ -195,10 +195,26 @@ def test_mid_tile_matches_small_tile(dev, policy, m, n, k, bs, od):
     assert _rel(out, ref + bias.double()) < (1e-4 if od == torch.float32 else 3e-3)
 
 
+@pytest.mark.parametrize("m,n,k,mid", [(1000, 4096, 1024, False), (1000, 4096, 1536, True),
+                                       (600, 4096, 1104, True), (500, 8192, 1408, False)])
+def test_mid_tile_one_round_line(dev, m, n, k, mid):
+    """Per tensor, in one round of the 128 x 128 tile: K from 1536 on, from 1024
+    where the operand rows do not start on 128-byte lines."""
+    g = torch.Generator().manual_seed(k)
+    a, sa = K.quantize_per_tensor(torch.randn(m, k, generator=g).to(dev))
+    hi, lo, ih, il = K.dual_quantize_per_tensor(torch.randn(n, k, generator=g).to(dev))
+    ref = (a.double() * sa.double()) @ (hi.double() * ih.double() + lo.double() * il.double()).t()
+
+    def run():
+        return K.fused_dual_gemm_forward(a, hi, lo, sa, ih, il)
+    assert any("4, 128, 128, " in s for s in _kernel_names(run)) == mid
+    assert _rel(run(), ref) < 1e-4
+
+
 # every tile a dgrad may take: the weight stream, one round of the small tile,
 # the 128 x 128 tile, the large one, the persistent one with eight and four waves
 @pytest.mark.parametrize("m,n,k", [(40, 520, 256), (300, 512, 400), (1000, 4096, 1024),
-                                   (8192, 1024, 384), (4096, 4096, 256), (2048, 4608, 8192)])
+                                   (1000, 4096, 1552), (8192, 1024, 384), (4096, 4096, 256), (2048, 4608, 8192)])
 def test_bf16_gradient_is_the_rounded_fp32_one(dev, m, n, k):
     g = torch.Generator().manual_seed(m + k)
     a, sa = K.quantize_per_tensor(torch.randn(m, k, generator=g).to(dev), E5M2)
