@@ -1199,7 +1199,9 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && NS == 2 && BM <= 128 ? 2 : 1))
   float c0s = 1.0f, c1s = 1.0f;
   if (SCALE == 0 && g.s_a) {
     const float sa = *g.s_a;
-    c0s = g.s_0 ? sa * *g.s_0 : sa;
+    // (the bf16 weight gradient's scale is one factor)
+    if constexpr (AF == kBF16) c0s = g.s_0 ? sa * *g.s_0 : sa;
+    else c0s = sa * *g.s_0;
     c1s = SPLIT ? c0s : sa * *g.s_1;
   }
   const bool vec = (g.ldo % (16 / EB)) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;

@@ -527,7 +527,6 @@ __global__ __launch_bounds__(kThreads) void amax_cand_kernel(const InT* __restri
     emit(&v, live ? 1 : 0);
   }
   __syncthreads();
-  __syncthreads();
   if (lane == 0) red[threadIdx.x >> 6] = wmin;
   __syncthreads();
   if (threadIdx.x == 0) {
