@@ -1,5 +1,5 @@
-"""Every GEMM kernel instantiation the C ABI can reach, held to a float64
-matmul of the same decoded operands.
+"""Every kernel instantiation that a product of FP8 operands reaches through
+the C ABI, held to a float64 matmul of the same decoded operands.
 
 ``tcfp_dual_gemm`` (per-tensor scales), ``tcfp_block_dual_gemm`` (int8
 block exponents on the MFMA's E8M0 scale operands) and
@@ -49,13 +49,25 @@ PATHS = {
     "persist_spl128": ("auto", (4096, 4096, 256), None),
     # per-tensor dual, bf16 output: the persistent tile with four waves
     "persist4": ("large4", BIG, None),
+    # block exponents through LDS, four stages: ragged on every side
+    "deep_exp": ("auto", (250, 260, 704), "4, 128, 64, {S}, 4, "),
+    # the 128 x 128 tile, three stages
+    "mid": ("mid", (250, 260, 320), "4, 128, 128, {S}, 3, "),
+    # the persistent tile on sizes that are no multiples of it
+    "ragged": ("auto", (4112, 2064, 320), None),
+    # up to 64 rows and E4M3 weights: the weight stream, 1, 2 or 4 row tiles
+    "stream1": ("auto", (13, 1000, 576), None),
+    "stream2": ("auto", (27, 1000, 576), None),
+    "stream4": ("auto", (61, 1000, 576), None),
 }
+STREAM = ["stream1", "stream2", "stream4"]
 # (scale kind, dual) -> the tile paths the dispatcher has for it
 SCALE_PATHS = {
-    ("pt", True): ["deep", "small8", "small2", "large", "persist", "persist4"],
-    ("pt", False): ["deep", "small8", "small2", "large"],
-    ("e8m0", True): ["small", "large", "persist"],
-    ("e8m0", False): ["small", "persist_spl", "persist_spl128"],
+    ("pt", True): ["deep", "small8", "small2", "large", "persist", "persist4", "mid", "ragged",
+                   *STREAM],
+    ("pt", False): ["deep", "small8", "small2", "large", *STREAM],
+    ("e8m0", True): ["small", "large", "persist", "deep_exp", "mid", "ragged", *STREAM],
+    ("e8m0", False): ["small", "persist_spl", "persist_spl128", "deep_exp", *STREAM],
     ("f32s", True): ["small"],
     ("f32s", False): ["small"],
 }
@@ -70,8 +82,10 @@ def _cases():
                 if path == "persist4" and od != "bf16":
                     continue
                 for af in (0, 1):
-                    for bf in (0, 1):
+                    for bf in (0,) if path in STREAM else (0, 1):
                         bss = (32, 64, 128) if kind == "f32s" else ((64,) if kind == "e8m0" else (0,))
+                        if kind == "e8m0" and path == "mid":
+                            bss = (32, 64)  # blocks of 128 run the kernel of 64
                         for bs in bss:
                             out.append(pytest.param(
                                 kind, bs, dual, path, od, af, bf,
@@ -160,13 +174,17 @@ def test_gemm_instantiation_against_float64(dev, kind, bs, dual, path, od, af, b
         want = f"gemm_nt_persist_kernel<{af}, {bf}, float, 0, 1, 6, 64, true>"
     elif path == "persist4":
         want = f"gemm_nt_persist_kernel<{af}, {bf}, unsigned short, 0, 0, 4, 128, false>"
+    elif path == "ragged":
+        want = f"gemm_nt_ragged_kernel<{af}, {bf}, {out_name}, {scale_id}>"
+    elif path in STREAM:
+        want = f"gemm_skinny_kernel<{af}, {bf}, {split}, {out_name}, {scale_id}, {path[-1]}>"
     elif path == "persist_spl128":
         want = f"gemm_nt_persist_kernel<{af}, {bf}, float, 0, 1, 8, 128, true>"
     elif frag is None:
         want = f"gemm_nt_persist_kernel<{af}, {bf}, {out_name}, 0, {scale_id}, 8, 128, false>"
     else:
         want = f"gemm_nt_dma_kernel<{af}, {bf}, {split}, {out_name}, " + frag.format(S=scale_id)
-        if kind == "f32s":
+        if kind == "f32s" or (kind == "e8m0" and path == "mid"):
             want += f"{bs.bit_length() - 1}, 0>"
     try:
         K.set_gemm_tile_policy(policy)

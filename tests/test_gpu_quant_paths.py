@@ -98,11 +98,57 @@ def test_candidate_windows_match_full_pass(dev, name, wdtype, ef):
         assert torch.equal(x, y)
 
 
+def _requests(monkeypatch, name, pick):
+    """What the layers ask of the op `name` from here on, by `pick`."""
+    seen, op = [], getattr(K, name)
+
+    def wrapped(*args, **kw):
+        seen.append(pick(*args, **kw))
+        return op(*args, **kw)
+
+    monkeypatch.setattr(K, name, wrapped)
+    return seen
+
+
+def _batch_copies(dual=(), act=()):
+    """(weights' transposed codes, activations' transposed codes) of a batch"""
+    return [t for *_, t in dual], [t for *_, t in act]
+
+
+def test_batched_layer_asks_for_backward_copies_only_when_recording(dev, monkeypatch):
+    seen = _requests(monkeypatch, "quantize_batch", _batch_copies)
+    layer = TCFPLinear(256, 256, use_tensor_cores=True).to(dev)
+    x = torch.randn(48, 256, device=dev, requires_grad=True)
+    layer(x)
+    with torch.no_grad():
+        layer(x)
+    assert seen == [([True], [True]), ([False], [False])]
+
+
+def test_mlp_asks_for_backward_copies_only_when_recording(dev, monkeypatch):
+    seen = _requests(monkeypatch, "quantize_batch", _batch_copies)
+    gelu = _requests(monkeypatch, "dual_gemm_gelu_quantize",
+                     lambda *a, transpose=False, return_dgelu=False, **kw: (transpose,
+                                                                            return_dgelu))
+    mlp = fuse_tcfp_mlp(torch.nn.Sequential(
+        TCFPLinear(256, 512, use_tensor_cores=True), torch.nn.GELU(),
+        TCFPLinear(512, 256, use_tensor_cores=True))).to(dev)
+    x = torch.randn(64, 256, device=dev, requires_grad=True)
+    mlp(x)
+    with torch.no_grad():
+        mlp(x)
+    assert gelu == [(True, True), (False, False)]
+    half = len(seen) // 2
+    assert all(all(w) and all(a) for w, a in seen[:half])
+    assert not any(any(w) or any(a) for w, a in seen[half:])
+
+
 @pytest.mark.parametrize("kw,d", [({}, 256), ({"scale_block_size": 64}, 1024), ({}, 2944)])
 def test_forward_without_autograd_makes_no_backward_copies(dev, kw, d):
     """Under no_grad: the values of the recording forward, no transposed codes
-    (d = 2944: the weight beyond the batch's size), parameters untouched, and
-    forward-mode AD still refused."""
+    (by kernel name at d = 2944, the weight beyond the batch's size, where a
+    kernel of its own writes them; the batch's are checked above), parameters
+    untouched, and forward-mode AD still refused."""
     torch.manual_seed(0)
     layer = TCFPLinear(d, d, use_tensor_cores=True, **kw).to(dev)
     x = torch.randn(48, d, device=dev, requires_grad=True)
