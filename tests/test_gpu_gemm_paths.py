@@ -223,7 +223,8 @@ def test_bf16_gradient_is_the_rounded_fp32_one(dev, m, n, k):
     assert torch.equal(K._dual_gemm(a, hi, lo, sa, ih, il, None, torch.bfloat16), f32.bfloat16())
 
 
-@pytest.mark.parametrize("m,n,k", [(100, 128, 192), (4096, 256, 1024), (2048, 4096, 8192)])
+@pytest.mark.parametrize("m,n,k", [(100, 128, 192), (4096, 256, 1024), (2048, 4096, 8192),
+                                   (4096, 2048, 4096)])
 def test_block_backward_bf16_gradient(dev, m, n, k):
     """block_linear_backward's dX in bf16 is its fp32 dX rounded (with W_lo, and
     W_hi alone), dW and db the same."""
