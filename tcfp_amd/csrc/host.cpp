@@ -54,6 +54,15 @@ struct Raise {
 struct Outs {
   std::vector<Tensor> t;
 };
+// (takes the caller's locals: a copy is two atomic counts, and a second owner
+// where Python's object is made)
+template <typename... T>
+Outs outs(T&... t) {
+  Outs o;
+  o.t.reserve(sizeof...(t));
+  (o.t.push_back(std::move(t)), ...);
+  return o;
+}
 
 std::string shape_str(at::IntArrayRef s) {
   std::string r = "(";
@@ -241,10 +250,10 @@ Outs quantize_per_tensor(const Tensor& x, at::ScalarType fp8, const OptT& scale,
   check(tcfp_quantize_per_tensor(ptr(v.t), dt, v.rows, v.cols, fmt, f32(s_in), bytes(q),
                                  bytes(q_t), f32(s_out), f32(inv), ws ? ws->ptr() : nullptr, st),
         "quantize_per_tensor");
-  if (transpose && return_scale) return {{q, inv, q_t, s_out}};
-  if (transpose) return {{q, inv, q_t}};
-  if (return_scale) return {{q, inv, s_out}};
-  return {{q, inv}};
+  if (transpose && return_scale) return outs(q, inv, q_t, s_out);
+  if (transpose) return outs(q, inv, q_t);
+  if (return_scale) return outs(q, inv, s_out);
+  return outs(q, inv);
 }
 
 Outs quantize_per_tensor_colsum(const Tensor& x, at::ScalarType fp8, bool transpose) {
@@ -263,8 +272,8 @@ Outs quantize_per_tensor_colsum(const Tensor& x, at::ScalarType fp8, bool transp
   check(tcfp_quantize_per_tensor_colsum(ptr(v.t), dt, v.rows, v.cols, fmt, bytes(q), bytes(q_t),
                                         f32(inv), f32(cs), ws.ptr(), ptr(cws), n, st),
         "quantize_per_tensor_colsum");
-  if (transpose) return {{q, inv, q_t, cs}};
-  return {{q, inv, cs}};
+  if (transpose) return outs(q, inv, q_t, cs);
+  return outs(q, inv, cs);
 }
 
 void check_ef(const Tensor& ef, int64_t n, int64_t k) {
@@ -299,8 +308,8 @@ Outs dual_quantize_per_tensor(const Tensor& weight, const OptT& error_buf, bool 
                                       stochastic_lo ? 1 : 0, seed, 0, bytes(hi), bytes(lo),
                                       f32(ih), f32(il), bytes(hi_t), bytes(lo_t), ws.ptr(), st),
         "dual_quantize_per_tensor");
-  if (transposed) return {{hi, lo, ih, il, hi_t, lo_t}};
-  return {{hi, lo, ih, il}};
+  if (transposed) return outs(hi, lo, ih, il, hi_t, lo_t);
+  return outs(hi, lo, ih, il);
 }
 
 // (weight, error_buf, update_ef, transposed) and (x, fp8_dtype, transpose)
@@ -351,8 +360,8 @@ std::pair<std::vector<Outs>, std::vector<Outs>> quantize_batch(const std::vector
     j.q_lo = bytes(lo);
     j.q_lo_t = bytes(lt);
     j.inv_lo = f32(il);
-    if (t) rd.push_back({{hi, lo, ih, il, ht, lt}});
-    else rd.push_back({{hi, lo, ih, il}});
+    if (t) rd.push_back(outs(hi, lo, ih, il, ht, lt));
+    else rd.push_back(outs(hi, lo, ih, il));
   }
   for (const auto& a : act) {
     Tensor x = std::get<0>(a);
@@ -374,13 +383,13 @@ std::pair<std::vector<Outs>, std::vector<Outs>> quantize_batch(const std::vector
     j.q = bytes(q);
     j.q_t = bytes(qt);
     j.inv = f32(inv);
-    if (std::get<2>(a)) ra.push_back({{q, inv, qt}});
-    else ra.push_back({{q, inv}});
+    if (std::get<2>(a)) ra.push_back(outs(q, inv, qt));
+    else ra.push_back(outs(q, inv));
   }
   void* st = g.stream();
   const Workspace ws(g, st, true);
   check(tcfp_quantize_batch(nj, jobs, ws.ptr(), ws.bytes(), st), "quantize_batch");
-  return {rd, ra};
+  return {std::move(rd), std::move(ra)};
 }
 
 // ---- GEMMs ----------------------------------------------------------------------
@@ -444,7 +453,7 @@ Outs block_quantize(const Tensor& x_, int64_t bs, at::ScalarType fp8, bool f32s)
                       : tcfp_block_quantize(ptr(x), dt, m, k, int(bs), fmt, bytes(q), exps(s),
                                             g.stream());
   check(rc, "block_quantize_fp8");
-  return {{q, s}};
+  return outs(q, s);
 }
 
 Tensor block_scales(const Tensor& e, int64_t rows, int64_t nkb, const char* name,
@@ -556,10 +565,10 @@ Outs dual_gemm_gelu_quantize(const Tensor& a_, const Tensor& b_hi_, const Tensor
             fmt_of(o.b_hi.scalar_type()), o.b_hi.stride(0), m, n, k, f32(sa), f32(sh), f32(sl),
             f32(b), f32(h), f32(act), f32(dg), fmt, bytes(q), bytes(q_t), f32(inv), ws.ptr(), st),
         "dual_gemm_gelu_quantize");
-  Outs r{{h, q, inv}};
-  if (transpose) r.t.push_back(q_t);
-  if (return_act) r.t.push_back(act);
-  if (return_dgelu) r.t.push_back(dg);
+  Outs r = outs(h, q, inv);
+  if (transpose) r.t.push_back(std::move(q_t));
+  if (return_act) r.t.push_back(std::move(act));
+  if (return_dgelu) r.t.push_back(std::move(dg));
   return r;
 }
 
@@ -600,10 +609,10 @@ Outs dual_gemm_dgelu_quantize_colsum(const Tensor& a_, const Tensor& b_hi_,
             f32(dc), f32(gr), fmt, bytes(q), bytes(q_t), f32(inv), f32(cs), ws.ptr(), ptr(cws),
             nbytes, st),
         "dual_gemm_dgelu_quantize_colsum");
-  Outs r{{q, inv}};
-  if (transpose) r.t.push_back(q_t);
-  if (col_sum) r.t.push_back(cs);
-  if (return_grad) r.t.push_back(gr);
+  Outs r = outs(q, inv);
+  if (transpose) r.t.push_back(std::move(q_t));
+  if (col_sum) r.t.push_back(std::move(cs));
+  if (return_grad) r.t.push_back(std::move(gr));
   return r;
 }
 
@@ -653,7 +662,7 @@ Outs block_linear_forward(const Tensor& x2d, const Tensor& weight, const OptT& b
                                ptr(out), TCFP_DTYPE_F32, N, st),
           "block_dual_gemm");
   }
-  return {{out, hi, lo, eh, el, aq, ae}};
+  return outs(out, hi, lo, eh, el, aq, ae);
 }
 
 // G^T deq(X) to fp32 accuracy for any token count: per-tensor codes with their
@@ -733,7 +742,7 @@ Outs block_linear_backward(const Tensor& grad_2d, const OptT& act_fp8, const Opt
                                           out_dtype_of(dx_dtype), ptr(ws), n, st),
           "block_dgrad_from_prep");
   }
-  return {{dx, dw, db}};
+  return outs(dx, dw, db);
 }
 
 }  // namespace
@@ -743,10 +752,13 @@ template <>
 struct type_caster<Outs> {
   PYBIND11_TYPE_CASTER(Outs, const_name("tuple"));
   bool load(handle, bool) { return false; }  // results only
-  static handle cast(const Outs& o, return_value_policy, handle) {
+  static handle cast(Outs&& o, return_value_policy, handle) {
     tuple r(o.t.size());
-    for (size_t i = 0; i < o.t.size(); ++i)
-      r[i] = o.t[i].defined() ? pybind11::cast(o.t[i]) : object(none());
+    for (size_t i = 0; i < o.t.size(); ++i) {
+      PyObject* t = THPVariable_Wrap(std::move(o.t[i]));
+      if (!t) throw error_already_set();
+      PyTuple_SET_ITEM(r.ptr(), ssize_t(i), t);
+    }
     return r.release();
   }
 };
