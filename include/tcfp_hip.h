@@ -659,7 +659,15 @@ int tcfp_transpose_u8(const uint8_t* src, int64_t rows, int64_t cols, uint8_t* d
  * small-tile grid fits in one round (FP8 operands; bf16 ones keep four
  * waves), 4 256 x 128 with one workgroup per tile (no persistent launch),
  * 5 the four-wave persistent 256 x 128 tile for per-tensor dual GEMMs with
- * bf16 output (the others as 0).  Results do not depend on the policy. */
+ * bf16 output and full tiles, more than CUs (the others 256 x 128), 6 128 x 128
+ * for dual GEMMs with per-tensor scales or block exponents (the others 256 x
+ * 128).  Block-scaled single GEMMs and fp32 block multipliers run 128 x 64
+ * wherever 256 x 128 is named, but for the former's persistent launches.
+ * 0 also takes 128 x 128 for dual GEMMs between one round of the
+ * small tile and one of the large, and for up to 64 rows a launch that streams
+ * the weights.  Policies 1 - 6 agree bit for bit, and so does 0 except where it
+ * streams: that launch sums K in another order, within the rounding of an fp32
+ * sum. */
 int tcfp_gemm_set_tile_policy(int policy);
 
 /* ---- self-test hooks (no reference counterpart) ------------------------ */

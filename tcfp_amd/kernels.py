@@ -822,8 +822,8 @@ def _lo_threshold(w_lo: torch.Tensor, lo_scales: torch.Tensor, threshold: float,
     reference's tile width is its autotuned ``BLOCK_N`` (64 or 128), so its
     result depends on the configuration it picked; this build fixes the
     rule at 64-row tiles.  Dropped blocks become zero codes under the
-    sentinel, which the GEMM skips.  Threshold <= 0 changes nothing (only
-    sentinel blocks qualify, and the GEMM skips wave tiles of those)."""
+    sentinel, under which they add nothing.  Threshold <= 0 changes nothing
+    (only sentinel blocks qualify)."""
     if threshold <= 0.0:
         return w_lo, lo_scales
     n = w_lo.shape[0]
@@ -880,8 +880,8 @@ def fused_block_scaled_dual_gemm_forward(
 
     Reference: ``fused_block_scaled_dual_gemm_forward``
     (``tcfp/kernels.py:1939-2028``).  W_lo exponents of -128 (zero residual
-    blocks) contribute nothing, and on the 128 x 64 tile a wave tile whose
-    W_lo exponents are all the sentinel skips its W_lo MFMAs (the
+    blocks) contribute nothing, and on the two-stage 128 x 64 tile a wave tile
+    whose W_lo exponents are all the sentinel skips its W_lo MFMAs (the
     reference's sparsity fast path at its default threshold 0).  ``sparse_threshold > 0`` drops the
     W_lo blocks the reference's rule drops (``_lo_threshold``).
     ``persistent`` and ``launch_mult`` are scheduling hints of the
@@ -1383,8 +1383,9 @@ def set_gemm_tile_policy(policy: str) -> None:
     the persistent launch), ``"large4"`` (the persistent 256 x 128 tile
     with four waves, one per SIMD, for per-tensor dual GEMMs with bf16
     output) or ``"mid"`` (128 x 128 tiles, four waves, three stages, for dual
-    GEMMs with per-tensor scales or block exponents).  Results do not depend
-    on the policy."""
+    GEMMs with per-tensor scales or block exponents).  The policies agree bit
+    for bit except where ``"auto"`` streams the weights (up to 64 rows), which
+    sums K in another order."""
     code = {"auto": 0, "large": 1, "small": 2, "small8": 3, "large_nonpersistent": 4,
             "large4": 5, "mid": 6}[policy]
     check(_hip.lib().tcfp_gemm_set_tile_policy(code), "set_gemm_tile_policy")
