@@ -684,12 +684,23 @@ Tensor wgrad_f32(const Tensor& grad, const Tensor& act, const OptT& inv, const O
   Tensor s, e;
   if (inv) s = scalar(*inv, "scale");
   if (act_e) e = block_scales(*act_e, m, bs > 0 ? k / bs : 0, "act_scales", at::kChar);
-  Tensor dw = g.empty({n, k}, at::kFloat);
-  const size_t nb = tcfp_wgrad_f32_workspace_bytes(m, n, k);
-  Tensor ws = g.empty({int64_t(std::max<size_t>(nb, 1))}, at::kByte);
-  check(tcfp_wgrad_f32(f32(gr), m, n, bytes(a), fmt_of(a.scalar_type()), f32(s), exps(e), k,
-                       int(bs), f32(dw), ptr(ws), nb, g.stream()),
-        "wgrad_f32");
+  // the GEMM's descriptors span a tile's rows of the split gradient, 6 bytes a
+  // token: sums of more tokens (1.4 million with its 256-row tile) are formed
+  // in runs of these and added
+  constexpr int64_t kTokens = int64_t(1) << 20;
+  Tensor dw;
+  for (int64_t r = 0; r < std::max<int64_t>(m, 1); r += kTokens) {
+    const int64_t c = std::min(kTokens, m - r);
+    const size_t nb = tcfp_wgrad_f32_workspace_bytes(c, n, k);
+    Tensor part = g.empty({n, k}, at::kFloat), er = e;
+    Tensor ws = g.empty({int64_t(std::max<size_t>(nb, 1))}, at::kByte);
+    if (e.defined() && c < m) er = e.narrow(1, r, c).contiguous();
+    check(tcfp_wgrad_f32(f32(gr) + r * n, c, n, bytes(a) + r * k, fmt_of(a.scalar_type()), f32(s),
+                         exps(er), k, int(bs), f32(part), ptr(ws), nb, g.stream()),
+          "wgrad_f32");
+    if (dw.defined()) dw.add_(part);
+    else dw = part;
+  }
   return dw;
 }
 

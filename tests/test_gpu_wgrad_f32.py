@@ -110,6 +110,25 @@ def test_layer_uses_it(dev):
     assert _rel(layer.weight.grad, ref) < 1e-6
 
 
+@pytest.mark.parametrize("bs", [0, 32])
+def test_millions_of_tokens(dev, bs):
+    """More tokens than one launch's descriptors span (2.8 million at the 128-row
+    tile), an odd number of them."""
+    m, n, k = 2_900_003, 16, 32
+    gen = torch.Generator(device=dev).manual_seed(3)
+    g = torch.randn(m, n, generator=gen, device=dev)
+    x = torch.randn(m, k, generator=gen, device=dev)
+    if bs:
+        q, e = K.block_quantize_fp8(x, bs)
+        dw, deq = K.block_scaled_wgrad(g, q, e, bs), K.block_dequantize_fp8(q, e, bs)
+    else:
+        q, inv = K.quantize_per_tensor(x)
+        dw, deq = K.wgrad_f32(g, q, inv), q.float() * inv
+    ref = g.double().t() @ deq.double()
+    # (sums of 2.9e6 terms that cancel to 1.7e3: the fp32 product's own error)
+    assert _rel(dw, ref) <= max(1.2 * _rel(g.t() @ deq, ref), 2e-7)
+
+
 @pytest.mark.parametrize("bs", [None, 32])
 def test_layer_under_create_graph(dev, bs):
     """A gradient penalty on dW at an odd token count: the weight gradient of a
